@@ -855,7 +855,7 @@ int spk_render_create(spk_scene* s, const spk_camera_desc* cam, const spk_render
     }
     if ((rc = r->hit.alloc(Q * 16)) || (rc = r->qs_o.alloc(Q * 16)) || (rc = r->qs_d.alloc(Q * 16)) ||
         (rc = r->qs_c.alloc(Q * 16)) || (rc = r->qm_o.alloc(Q * 16)) || (rc = r->qm_d.alloc(Q * 16)) ||
-        (rc = r->qm_c.alloc(Q * 16)) || (rc = r->path_L.alloc((size_t)r->capacity * 16)))
+        (rc = r->qm_c.alloc(Q * 16)) || (rc = r->path_L.alloc(std::max<size_t>((size_t)r->capacity * 16, 64))))  // 64: film read-back, one pixel
         return rc;
     if (regen) {
         SPK_CHECK_HIP(hipHostMalloc((void**)&r->rg_flag, 2 * sizeof(uint32_t), hipHostMallocDefault));
@@ -1153,6 +1153,30 @@ int run_passes(spk_render* r, int64_t first, int32_t n_spp, const GuideNetDev* n
     return SPK_OK;
 }
 
+// Film read-back goes through the path radiance slots: they hold nothing between passes (a pass
+// starts by clearing its own, and everything here is ordered on the render's stream), so no
+// workspace is allocated.  Pixels a read-back resolves at a time, at `bytes` each.
+size_t film_chunk(const spk_render* r, size_t bytes) {
+    return std::max<size_t>(1, std::min<size_t>(r->path_L.bytes / bytes, size_t(1) << 28));
+}
+
+// Film pixels [off, off + P) as the caller's float64 sums and counts (any pointer may be null).
+int film_download(spk_render* r, size_t off, size_t P, double* sum_rgb, double* sumsq_rgb, double* count) {
+    const size_t chunk = film_chunk(r, 56);
+    for (size_t p0 = 0; p0 < P; p0 += chunk) {
+        const size_t n = std::min(chunk, P - p0);
+        double* d = r->path_L.as<double>();
+        double *ds = sum_rgb ? d : nullptr, *dq = sumsq_rgb ? d + 3 * n : nullptr, *dc = count ? d + 6 * n : nullptr;
+        int rc;
+        if ((rc = launch_resolve_film(r->bufs, off + p0, (uint32_t)n, ds, dq, dc, r->stream))) return rc;
+        if (ds) SPK_CHECK_HIP(hipMemcpyAsync(sum_rgb + 3 * p0, ds, n * 24, hipMemcpyDeviceToHost, r->stream));
+        if (dq) SPK_CHECK_HIP(hipMemcpyAsync(sumsq_rgb + 3 * p0, dq, n * 24, hipMemcpyDeviceToHost, r->stream));
+        if (dc) SPK_CHECK_HIP(hipMemcpyAsync(count + p0, dc, n * 8, hipMemcpyDeviceToHost, r->stream));
+        SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
+    }
+    return SPK_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1258,39 +1282,22 @@ int spk_render_film(spk_render* r, double* sum_rgb, double* sumsq_rgb, double* c
     clear_error();
     if (!r) return SPK_ERR_INVALID;
     SPK_CHECK_HIP(hipSetDevice(r->device));
-    SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
-    size_t P = r->cfg.npix;
-    std::vector<float4> s(P), c(P), q(P), qc(P);
-    SPK_CHECK_HIP(hipMemcpy(s.data(), r->film_sum.p, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(c.data(), r->film_c.p, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(q.data(), r->film_sq.p, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(qc.data(), r->film_sqc.p, P * 16, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < P; i++) {
-        // The Kahan compensation holds the negated lost low-order part.
-        if (sum_rgb) {
-            sum_rgb[3 * i] = (double)s[i].x - (double)c[i].x;
-            sum_rgb[3 * i + 1] = (double)s[i].y - (double)c[i].y;
-            sum_rgb[3 * i + 2] = (double)s[i].z - (double)c[i].z;
-        }
-        if (sumsq_rgb) {
-            sumsq_rgb[3 * i] = (double)q[i].x - (double)qc[i].x;
-            sumsq_rgb[3 * i + 1] = (double)q[i].y - (double)qc[i].y;
-            sumsq_rgb[3 * i + 2] = (double)q[i].z - (double)qc[i].z;
-        }
-        if (count) count[i] = (double)s[i].w;
-    }
-    return SPK_OK;
+    return film_download(r, 0, r->cfg.npix, sum_rgb, sumsq_rgb, count);
 }
 
 int spk_render_image(spk_render* r, float* rgb) {
     clear_error();
     if (!r || !rgb) return SPK_ERR_INVALID;
-    size_t P = r->cfg.npix;
-    std::vector<double> sum(P * 3), cnt(P);
-    int rc = spk_render_film(r, sum.data(), nullptr, cnt.data());
-    if (rc) return rc;
-    for (size_t i = 0; i < P; i++)
-        for (int k = 0; k < 3; k++) rgb[3 * i + k] = (float)(sum[3 * i + k] / (cnt[i] + 1e-12));
+    SPK_CHECK_HIP(hipSetDevice(r->device));
+    const size_t P = r->cfg.npix, chunk = film_chunk(r, 12);
+    for (size_t p0 = 0; p0 < P; p0 += chunk) {
+        const uint32_t n = (uint32_t)std::min(chunk, P - p0);
+        float* d = r->path_L.as<float>();
+        int rc;
+        if ((rc = launch_resolve_image(r->bufs, p0, n, d, r->stream))) return rc;
+        SPK_CHECK_HIP(hipMemcpyAsync(rgb + 3 * p0, d, (size_t)n * 12, hipMemcpyDeviceToHost, r->stream));
+        SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
+    }
     return SPK_OK;
 }
 
@@ -1768,28 +1775,8 @@ int spk_batch_film(spk_batch* b, int32_t image, double* sum_rgb, double* sumsq_r
     if (!b || image < 0 || image >= (int32_t)b->images.size()) return SPK_ERR_INVALID;
     spk_render* r = b->r;
     SPK_CHECK_HIP(hipSetDevice(r->device));
-    SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
     const ImageDev& im = b->images[image];
-    const size_t P = (size_t)im.cam.W * im.cam.H, off = im.film_off;
-    std::vector<float4> s(P), c(P), q(P), qc(P);
-    SPK_CHECK_HIP(hipMemcpy(s.data(), r->film_sum.as<float4>() + off, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(c.data(), r->film_c.as<float4>() + off, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(q.data(), r->film_sq.as<float4>() + off, P * 16, hipMemcpyDeviceToHost));
-    SPK_CHECK_HIP(hipMemcpy(qc.data(), r->film_sqc.as<float4>() + off, P * 16, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < P; i++) {
-        if (sum_rgb) {
-            sum_rgb[3 * i] = (double)s[i].x - (double)c[i].x;
-            sum_rgb[3 * i + 1] = (double)s[i].y - (double)c[i].y;
-            sum_rgb[3 * i + 2] = (double)s[i].z - (double)c[i].z;
-        }
-        if (sumsq_rgb) {
-            sumsq_rgb[3 * i] = (double)q[i].x - (double)qc[i].x;
-            sumsq_rgb[3 * i + 1] = (double)q[i].y - (double)qc[i].y;
-            sumsq_rgb[3 * i + 2] = (double)q[i].z - (double)qc[i].z;
-        }
-        if (count) count[i] = (double)s[i].w;
-    }
-    return SPK_OK;
+    return film_download(r, im.film_off, (size_t)im.cam.W * im.cam.H, sum_rgb, sumsq_rgb, count);
 }
 
 int spk_batch_info_get(spk_batch* b, spk_batch_info* out) {

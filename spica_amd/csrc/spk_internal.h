@@ -197,6 +197,10 @@ int launch_regen_end(const RenderBufs& b, const ConfigDev& cfg, const LaunchShap
                      int last_slot, const GuideNetDev* guide);
 int launch_set_pass(PassState* ps, uint32_t index, hipStream_t st);
 int launch_clear_film(const RenderBufs& b, uint32_t npix, hipStream_t st);
+// Film pixels [off, off + n) resolved into device arrays (spk_film.hip; any film output may be null).
+int launch_resolve_film(const RenderBufs& b, size_t off, uint32_t n, double* out_sum, double* out_sq, double* out_count,
+                        hipStream_t st);
+int launch_resolve_image(const RenderBufs& b, size_t off, uint32_t n, float* rgb, hipStream_t st);
 int launch_relmse(const RenderBufs& b, const ConfigDev& cfg, const double* ref, double eps, double* out_partial,
                   int nblocks, hipStream_t st);
 int launch_relmse_pixels(const RenderBufs& b, int64_t n, const int32_t* pixels, const double* ref, double eps,

@@ -1,0 +1,30 @@
+"""Film read-back: the image is the film's mean in float64 rounded to float32, and any subset of
+the film's arrays may be asked for, at the sizes where the read-back is cut differently (one
+pixel; one sample, where a film takes several pieces; many samples, where it takes one)."""
+import numpy as np
+import pytest
+
+from spica_amd import _abi, configs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (7, 1, 1), (61, 47, 1), (256, 3, 5)])
+def test_image_is_the_film_mean(gpu, w, h, spp):
+    wl = configs.cornell_box(width=w, height=h, spp=spp)
+    gs = gpu.GpuScene(wl.scene)
+    gr = gpu.GpuRender(gs, wl.camera, wl.render_desc())
+    gr.run(spp)
+    s, q, c = gr.film()
+    assert np.all(c == spp) and np.all(q >= 0)
+    assert np.array_equal(gr.image(), (s / (c[..., None] + 1e-12)).astype(np.float32))
+    assert w * h < 9 or s.sum() > 0
+    only = np.zeros_like(q)
+    lib = _abi.load()
+    assert lib.spk_render_film(gr.handle, None, only.ctypes.data_as(_abi.c_d_p), None) == 0
+    assert np.array_equal(only, q)
+    gr.run(spp)  # the read-back leaves nothing behind for the next samples
+    s2, _, c2 = gr.film()
+    ref = gpu.GpuRender(gs, wl.camera, wl.render_desc(spp=2 * spp))
+    ref.run(2 * spp)
+    assert np.array_equal(s2, ref.film()[0]) and np.all(c2 == 2 * spp)
