@@ -59,6 +59,15 @@ int zero_u32(uint32_t* p, int n, hipStream_t st);
 constexpr int64_t kRegenPassPaths = int64_t(1) << SPK_REGEN_PASS_LOG2;
 // Iterations of a regenerating pass launched between polls of its done flag.
 constexpr int kRegenGroup = 4;
+constexpr int kRegenGroupNear = 2;  // and near the end of a pass
+// Paths a pass's tail kernel takes at most.  Below it an iteration of the stage kernels is bound by
+// its longest rays (~190 us an iteration on a 200-sphere field at 20,000 paths as at 100,000), above
+// it by throughput, where the stage kernels' occupancy is better.  Microseconds a pass by limit,
+// 0 (never) / 2^14 / 2^16 / 2^18 / 2^20: every material under a sky, 805 k paths 4116 / 2301 / 1926 /
+// 1928 / 2082; guided 640x360x96 36646 / 31431 / 31248 / 29728 / 29792; 1920x1080x32 field
+// 29940 / 29954 / 28063 / 27524 / 27104; 8-image batch 18281 / 16962 / 16628 / 16255 / 16247;
+// 64x64x4 preview 634 / 231 / 210 / 209 / 210.
+constexpr uint32_t kTailMaxPaths = 1u << 18;
 int launch_sampler(int kind, uint32_t seed, int64_t n, const uint32_t* px, const uint32_t* sm, const uint32_t* dm,
                    uint32_t* out, hipStream_t st);
 
@@ -269,7 +278,7 @@ struct spk_render {
     DevBuf film_sum, film_c, film_sq, film_sqc, spill, cfg_dev, ps_dev, scratch;
     uint32_t capacity = 0;          // paths per pass (path radiance slots)
     uint32_t inflight = 0;          // queue capacity: = capacity for classic passes
-    uint32_t* rg_flag = nullptr;    // regen: pinned host words the done flag is copied to
+    uint32_t* rg_flag = nullptr;    // regen: pinned host words the (done, near the end) flags are copied to
     hipEvent_t rg_ev[2] = {nullptr, nullptr};
     hipGraphExec_t rg_exec = nullptr;  // use_graph with regen: one captured group of iterations
     int64_t rg_iterations = 0;      // regen iterations launched
@@ -846,6 +855,8 @@ int spk_render_create(spk_scene* s, const spk_camera_desc* cam, const spk_render
     c.seed = desc->seed;
     c.integrator = desc->integrator;
     c.wide = s->dev.wide;
+    // counting visits is the stage kernels' affair
+    c.tail_max = regen && o.count_visits == 0 ? kTailMaxPaths : 0;
 
     // Buffers: queues hold the paths in flight, path radiance every path of a pass.
     int rc;
@@ -858,8 +869,8 @@ int spk_render_create(spk_scene* s, const spk_camera_desc* cam, const spk_render
         (rc = r->qm_c.alloc(Q * 16)) || (rc = r->path_L.alloc(std::max<size_t>((size_t)r->capacity * 16, 64))))  // 64: film read-back, one pixel
         return rc;
     if (regen) {
-        SPK_CHECK_HIP(hipHostMalloc((void**)&r->rg_flag, 2 * sizeof(uint32_t), hipHostMallocDefault));
-        r->rg_flag[0] = r->rg_flag[1] = 0;
+        SPK_CHECK_HIP(hipHostMalloc((void**)&r->rg_flag, 4 * sizeof(uint32_t), hipHostMallocDefault));
+        memset(r->rg_flag, 0, 4 * sizeof(uint32_t));
         for (hipEvent_t& e : r->rg_ev) SPK_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     size_t P = c.npix;
@@ -872,6 +883,9 @@ int spk_render_create(spk_scene* s, const spk_camera_desc* cam, const spk_render
     r->shape.grid_trace = prop.multiProcessorCount * std::max(1, trace_blocks_per_cu(o.block_size));
     r->shape.grid_stream = prop.multiProcessorCount * 8;
     r->shape.grid_guide = prop.multiProcessorCount;
+    // one spill area per thread: no more tail threads than traversal threads
+    r->shape.grid_tail = std::min(prop.multiProcessorCount * tail_waves_per_cu(),
+                                  std::max(1, r->shape.grid_trace * o.block_size / 64));
     if ((rc = r->spill.alloc((size_t)r->shape.grid_trace * o.block_size * s->spill_cap * 4))) return rc;
     if ((rc = r->cfg_dev.alloc(sizeof(ConfigDev))) || (rc = r->ps_dev.alloc(sizeof(PassState)))) return rc;
     if ((rc = r->scratch.alloc(4096 * sizeof(double)))) return rc;
@@ -977,12 +991,16 @@ int ensure_events(spk_render* r, size_t need) {
 // at the end).  With use_graph one captured group (an even number of iterations, so every group
 // has the same queue slots) is replayed.  Profile events are appended from index *ev_next.
 int run_pass_regen(spk_render* r, const SceneDev& sd, bool batch, bool use_graph, const GuideNetDev* net,
-                   size_t* ev_next) {
+                   size_t* ev_next, uint64_t n_paths) {
     int rc;
     if ((rc = launch_regen_begin(r->bufs, batch, r->stream))) return rc;
     const bool prof = r->opts.profile != 0 && ev_next;
     const bool count = r->opts.count_visits != 0;
-    static_assert(kRegenGroup % 2 == 0, "a group keeps the slot pattern");
+    if (n_paths > 0 && n_paths <= std::min(r->cfg.tail_max, r->inflight) && !net && !prof) {
+        if ((rc = launch_regen_small(sd, r->bufs, r->cfg, r->shape, r->stream, batch, (uint32_t)n_paths))) return rc;
+        return launch_regen_end(r->bufs, r->cfg, r->shape, r->stream, batch, 0, net);
+    }
+    static_assert(kRegenGroup % 2 == 0 && kRegenGroupNear % 2 == 0, "a group keeps the slot pattern");
     // Every queued path advances one bounce per iteration and ends after maxDepth + 1, and an
     // iteration starts new paths whenever the queue has room, so a pass needs at most this many
     // iterations; beyond it something is wrong and the pass is abandoned with an error.
@@ -990,7 +1008,10 @@ int run_pass_regen(spk_render* r, const SceneDev& sd, bool batch, bool use_graph
     const int64_t max_it = (cap_paths / std::max<uint32_t>(r->inflight, 1) + 2) * (r->cfg.max_depth + 2) +
                            4 * kRegenGroup;
     int64_t it = 0;
+    // every path starts in the first iteration: the pass may be near its end after any group
+    bool near = n_paths <= r->inflight;
     for (int g = 0;; g++) {
+        const int n_it = near && !use_graph ? kRegenGroupNear : kRegenGroup;
         if (it > max_it) {
             SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
             set_error("regenerating pass did not finish after %lld iterations", (long long)it);
@@ -1013,21 +1034,26 @@ int run_pass_regen(spk_render* r, const SceneDev& sd, bool batch, bool use_graph
         } else {
             hipEvent_t* ev = nullptr;
             if (prof) {
-                if ((rc = ensure_events(r, *ev_next + 8 * kRegenGroup))) return rc;
+                if ((rc = ensure_events(r, *ev_next + 8 * (size_t)n_it))) return rc;
                 ev = &r->events[*ev_next];
-                *ev_next += 8 * kRegenGroup;
+                *ev_next += 8 * (size_t)n_it;
             }
-            if ((rc = launch_regen_iters(sd, r->bufs, r->cfg, r->shape, r->stream, batch, (int)it, kRegenGroup, ev,
+            if ((rc = launch_regen_iters(sd, r->bufs, r->cfg, r->shape, r->stream, batch, (int)it, n_it, ev,
                                          r->opts.profile >= 2 ? 8 : 2, count, net)))
                 return rc;
         }
-        it += kRegenGroup;
-        SPK_CHECK_HIP(hipMemcpyAsync(&r->rg_flag[g & 1], &r->bufs.ps->rg_done, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                     r->stream));
+        it += n_it;
+        SPK_CHECK_HIP(hipMemcpyAsync(&r->rg_flag[2 * (g & 1)], &r->bufs.ps->rg_done, 2 * sizeof(uint32_t),
+                                     hipMemcpyDeviceToHost, r->stream));
         SPK_CHECK_HIP(hipEventRecord(r->rg_ev[g & 1], r->stream));
-        if (g >= 1) {
+        if (g >= 1 && !near) {
             SPK_CHECK_HIP(hipEventSynchronize(r->rg_ev[(g - 1) & 1]));
-            if (r->rg_flag[(g - 1) & 1]) break;
+            if (r->rg_flag[2 * ((g - 1) & 1)]) break;
+            near = r->rg_flag[2 * ((g - 1) & 1) + 1] != 0;
+        }
+        if (near) {
+            SPK_CHECK_HIP(hipEventSynchronize(r->rg_ev[g & 1]));
+            if (r->rg_flag[2 * (g & 1)]) break;
         }
     }
     r->rg_iterations += it;
@@ -1071,25 +1097,30 @@ int run_passes(spk_render* r, int64_t first, int32_t n_spp, const GuideNetDev* n
     // per depth: start/end of the closest-hit, guide (guided renders), shade and shadow launches
     const int nd = c.max_depth + 1;
     int nev = 8 * nd;
+    // rays of the timed launches: the tail kernel's are not among them
     int64_t ext_before = 0, shadow_before = 0;
     if (r->opts.profile) {
         PassState ps;
         SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
         SPK_CHECK_HIP(hipMemcpy(&ps, r->ps_dev.p, sizeof(PassState), hipMemcpyDeviceToHost));
-        ext_before = (int64_t)ps.total_extend;
-        shadow_before = (int64_t)ps.total_shadow;
+        ext_before = (int64_t)(ps.total_extend - ps.tail_extend);
+        shadow_before = (int64_t)(ps.total_shadow - ps.tail_shadow);
         if (!c.regen && (rc = ensure_events(r, (size_t)passes * nev))) return rc;
     }
     if (c.regen) {
         size_t ev_next = 0;
-        for (int64_t p = 0; p < passes; p++)
-            if ((rc = run_pass_regen(r, r->scene->dev, false, r->opts.use_graph != 0, net, &ev_next))) return rc;
+        for (int64_t p = 0; p < passes; p++) {
+            const uint64_t n_paths =
+                c.chunks > 1 ? std::min<uint64_t>(c.queue, c.npix - (uint64_t)(p % c.chunks) * c.queue)
+                             : (uint64_t)c.npix * (uint64_t)std::min<int64_t>(c.kmax, n_spp - p * (int64_t)c.kmax);
+            if ((rc = run_pass_regen(r, r->scene->dev, false, r->opts.use_graph != 0, net, &ev_next, n_paths))) return rc;
+        }
         if (r->opts.profile) {
             SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
             PassState ps;
             SPK_CHECK_HIP(hipMemcpy(&ps, r->ps_dev.p, sizeof(PassState), hipMemcpyDeviceToHost));
-            r->extend_rays_timed += (int64_t)ps.total_extend - ext_before;
-            r->shadow_rays_timed += (int64_t)ps.total_shadow - shadow_before;
+            r->extend_rays_timed += (int64_t)(ps.total_extend - ps.tail_extend) - ext_before;
+            r->shadow_rays_timed += (int64_t)(ps.total_shadow - ps.tail_shadow) - shadow_before;
             if ((rc = regen_profile(r, (int64_t)(ev_next / 8), net != nullptr))) return rc;
         }
         return SPK_OK;
@@ -1720,7 +1751,7 @@ int spk_batch_run(spk_batch* b, int32_t sync) {
                 return rc;
             GuideNetDev net = guide_net(r, train);
             net.rec_keep = 1.0f / (float)g->opts.train_pass_spp;
-            if (r->cfg.regen) rc = run_pass_regen(r, *sd, true, false, &net, nullptr);
+            if (r->cfg.regen) rc = run_pass_regen(r, *sd, true, false, &net, nullptr, b->passes[p].n_paths);
             else rc = launch_batch_pass(r->bufs, r->cfg, r->shape, r->stream, sd, &net);
             if (rc) return rc;
             if (train && (p + 1 == np || b->pass_round[p + 1] != rd)) {
@@ -1740,7 +1771,7 @@ int spk_batch_run(spk_batch* b, int32_t sync) {
         if ((rc = launch_clear_film(r->bufs, (uint32_t)b->film_pixels, r->stream))) return rc;
         if ((rc = launch_set_pass(r->bufs.ps, 0, r->stream))) return rc;
         for (size_t p = 0; p < b->passes.size(); p++)
-            if ((rc = run_pass_regen(r, none, true, b->graph != 0, nullptr, nullptr))) return rc;
+            if ((rc = run_pass_regen(r, none, true, b->graph != 0, nullptr, nullptr, b->passes[p].n_paths))) return rc;
         r->samples_done++;
         if (sync) SPK_CHECK_HIP(hipStreamSynchronize(r->stream));
         return SPK_OK;

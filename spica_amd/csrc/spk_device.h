@@ -132,6 +132,7 @@ struct ConfigDev {
     uint32_t inflight;      // regen: queue capacity (paths in flight); the pass holds up to `queue`
     float guide_min_alpha;  // guided renders: microfacet reflections below this alpha are not guided
     int guide_depth;        // guided renders: vertices of bounces 0 .. guide_depth - 1 are guided
+    uint32_t tail_max;      // regen: the last tail_max paths of a pass go to the tail kernel (0: none do)
 };
 
 // Device-side per-pass state: queue lengths and work counters per bounce.
@@ -170,7 +171,13 @@ struct PassState {
     // regen: per iteration, the continuations carried over (n_cont), the new camera paths
     // appended after them (m_new, path ids from first_new), the next unstarted path of the
     // pass, the extend count, and done = no work left in this iteration
-    uint32_t rg_next, rg_ncont, rg_mnew, rg_first, rg_nin, rg_done, rg_pad[2];
+    uint32_t rg_next, rg_ncont, rg_mnew, rg_first, rg_nin;
+    uint32_t rg_done, rg_near;       // copied to the host together: no work left; few paths left
+    uint32_t rg_age;                 // iterations since the last camera path started
+    // the paths handed to the tail kernel (0: none) and the queue slot that holds them
+    uint32_t tail_n, tail_slot;
+    unsigned long long tail_extend;  // closest-hit and occlusion rays traced by the tail kernel
+    unsigned long long tail_shadow;
 };
 
 }  // namespace spk

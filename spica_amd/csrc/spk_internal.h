@@ -134,6 +134,7 @@ struct TraceBufs {
 int launch_trace(const SceneDev& s, const TraceBufs& b, uint32_t* work_counter, uint32_t* spill, int spill_cap,
                  int grid, hipStream_t st);
 int trace_blocks_per_cu(int block);
+int tail_waves_per_cu();
 // What a trace needs from a scene handle (the handle's layout is private to spk_api.cpp).
 struct SceneTraceInfo {
     const SceneDev* dev;
@@ -177,6 +178,7 @@ struct RenderBufs {
 struct LaunchShape {
     int grid_trace;     // persistent traversal blocks
     int grid_stream;    // grid-stride blocks for shading / streaming kernels
+    int grid_tail;      // tail-kernel blocks (one wave each)
     int grid_guide;     // persistent blocks of the guide kernel (one per CU)
     int block;          // threads per block
 };
@@ -193,6 +195,9 @@ int launch_regen_begin(const RenderBufs& b, bool batch, hipStream_t st);
 int launch_regen_iters(const SceneDev& s, const RenderBufs& b, const ConfigDev& cfg, const LaunchShape& ls,
                        hipStream_t st, bool batch, int it0, int n_it, hipEvent_t* ev, int ev_per_it, bool count,
                        const GuideNetDev* guide);
+// A pass of n_paths paths, few enough for the tail kernel alone: no iterations.
+int launch_regen_small(const SceneDev& s, const RenderBufs& b, const ConfigDev& cfg, const LaunchShape& ls, hipStream_t st,
+                       bool batch, uint32_t n_paths);
 int launch_regen_end(const RenderBufs& b, const ConfigDev& cfg, const LaunchShape& ls, hipStream_t st, bool batch,
                      int last_slot, const GuideNetDev* guide);
 int launch_set_pass(PassState* ps, uint32_t index, hipStream_t st);

@@ -1,0 +1,55 @@
+"""The tail kernel (the last paths of a pass, each to its end in one launch): films and ray counts equal
+those of classic passes, which never use it, bit for bit.  Sizes: one path, a wave's slice and one
+more, the most paths a pass may run without iterations, and one row more (iterations first, then the
+tail); every BSDF under a sky, the basic ones under area lights, direct lighting, a guided render."""
+import numpy as np
+import pytest
+
+from spica_amd import _abi, configs
+
+pytestmark = pytest.mark.gpu
+
+
+def _workload(kind, w, h, spp):
+    if kind == "sky":
+        scene, _ = configs.sphere_field(5, 40, mix=configs.WIDE_MIX)
+        scene.set_envmap(configs.sky_envmap(64, 32, sun=200.0),
+                         to_world=np.array([[1, 0, 0, 0], [0, 0, 1, 0], [0, 1, 0, 0], [0, 0, 0, 1]], float), radius=40.0)
+        cam = configs.c1_spheres(w, h, n_spheres=0).camera
+        return configs.Workload("sky", scene, cam, spp, 16, _abi.SPK_SAMPLER_SOBOL, 3)
+    return configs.c1_spheres(w, h, spp, n_spheres=60)
+
+
+def _render(gpu, gs, wl, spp, regen, integrator=None, guide=None):
+    gr = gpu.GpuRender(gs, wl.camera, wl.render_desc(integrator=integrator), regen=regen, queue_size=1 << 20)
+    if guide is not None:
+        gr.set_guide(guide)
+    gr.run(spp)
+    out = gr.film(), gr.stats()
+    gr.close()
+    return out
+
+
+@pytest.mark.parametrize("kind,integrator", [("field", "path"), ("sky", "path"), ("field", "direct")])
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (16, 1, 1), (17, 1, 1), (61, 47, 3), (512, 512, 1), (512, 513, 1)])
+def test_tail_equals_classic_passes(gpu, kind, integrator, w, h, spp):
+    wl = _workload(kind, w, h, spp)
+    gs = gpu.GpuScene(wl.scene)
+    integ = _abi.SPK_INTEGRATOR_DIRECT if integrator == "direct" else None
+    (s, q, c), st = _render(gpu, gs, wl, spp, True, integ)
+    (s0, q0, c0), st0 = _render(gpu, gs, wl, spp, False, integ)
+    assert np.array_equal(c, c0) and np.array_equal(s, s0) and np.array_equal(q, q0)
+    for key in ("paths", "rays_extend", "rays_shadow", "rays_mis"):
+        assert st[key] == st0[key], key
+
+
+def test_guided_tail_equals_classic_passes(gpu):
+    wl = configs.c3_occluded_glossy(width=300, height=200, n_spheres=64)
+    gs = gpu.GpuScene(wl.scene)
+    res = []
+    for regen in (True, False):
+        g = gpu.Guide(batch_size=1 << 14, train_spp=8, train_pass_spp=4, steps_per_pass=2)
+        res.append(_render(gpu, gs, wl, 12, regen, guide=g))
+    (f, st), (f0, st0) = res
+    assert all(np.array_equal(a, b) for a, b in zip(f, f0))
+    assert st["guided_vertices"] == st0["guided_vertices"] > 0 and st["rays_extend"] == st0["rays_extend"]
