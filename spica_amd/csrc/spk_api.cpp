@@ -242,7 +242,7 @@ struct spk_scene {
     SceneDev dev;
     DevBuf nodes, tris, tri_ng, tri_ids, tri_n, mats, lights;
     DevBuf env_tex, env_marg_cdf, env_marg_pdf, env_cond_cdf, env_cond_pdf, env_pdf2d;
-    DevBuf trace_work, trace_spill;
+    DevBuf trace_spill;
     int trace_grid = 0;
     int spill_cap = 0;
     float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {1.0f, 1.0f, 1.0f};  // bounding box of the triangles
@@ -713,7 +713,7 @@ int spk_scene_destroy(spk_scene* s) {
     (void)hipDeviceSynchronize();
     DevBuf* bufs[] = {&s->nodes, &s->tris, &s->tri_ng, &s->tri_ids, &s->tri_n, &s->mats, &s->lights,
                       &s->env_tex, &s->env_marg_cdf, &s->env_marg_pdf, &s->env_cond_cdf, &s->env_cond_pdf,
-                      &s->env_pdf2d, &s->trace_work, &s->trace_spill};
+                      &s->env_pdf2d, &s->trace_spill};
     for (DevBuf* b : bufs) b->release();
     delete s;
     return SPK_OK;
@@ -754,14 +754,12 @@ int spk_trace(spk_scene* s, const float* org, const float* dir, const float* tma
     SPK_CHECK_HIP(hipSetDevice(s->device));
     hipStream_t st = (hipStream_t)stream;
     int rc;
-    if (!s->trace_work.p) {
+    if (!s->trace_spill.p) {
         hipDeviceProp_t prop;
         SPK_CHECK_HIP(hipGetDeviceProperties(&prop, s->device));
         s->trace_grid = prop.multiProcessorCount * std::max(1, trace_blocks_per_cu(128));
-        if ((rc = s->trace_work.alloc(64))) return rc;
         if ((rc = s->trace_spill.alloc((size_t)s->trace_grid * 128 * s->spill_cap * 4))) return rc;
     }
-    if ((rc = zero_u32(s->trace_work.as<uint32_t>(), 16, st))) return rc;
     TraceBufs b;
     b.org = org;
     b.dir = dir;
@@ -770,8 +768,7 @@ int spk_trace(spk_scene* s, const float* org, const float* dir, const float* tma
     b.t_out = t_out;
     b.n = n;
     b.any_hit = any_hit ? 1 : 0;
-    return launch_trace(s->dev, b, s->trace_work.as<uint32_t>(), s->trace_spill.as<uint32_t>(), s->spill_cap,
-                        s->trace_grid, st);
+    return launch_trace(s->dev, b, s->trace_spill.as<uint32_t>(), s->spill_cap, s->trace_grid, st);
 }
 
 int spk_render_create(spk_scene* s, const spk_camera_desc* cam, const spk_render_desc* desc, const spk_render_opts* opts,

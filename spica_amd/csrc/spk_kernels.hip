@@ -7,14 +7,15 @@
 //   pass_init -> camera -> [extend -> shade -> shadow -> mis] x (maxDepth+1) -> film
 //
 // * extend / shadow / mis: persistent BVH traversal (closest hit / any hit /
-//   closest hit), rays pulled 64 at a time per wave from an atomic work counter,
-//   short per-lane stack in LDS (spilling to HBM only when a ray goes deeper than
-//   the LDS slots), interior-node loop with postponed leaves that the wave leaves
-//   only when every lane holds a leaf (wave vote).
+//   closest hit) over fixed slices of the queue, finished lanes taking the slice's next
+//   ray; short per-lane stack in LDS (spilling to HBM only when a ray goes deeper than
+//   the LDS slots), interior-node loop with one postponed leaf per lane that the wave
+//   leaves when few of its lanes have nodes left to visit (Walker).
 // * shade: one entry per hit; emission, spica's NEE (light sample + BSDF sample
 //   with the power heuristic, mis.cc:21-136), BSDF continuation and Russian
 //   roulette; it appends to the next extend queue, the shadow queue and the MIS
-//   queue with one atomic per wave per queue (ballot + mbcnt prefix).
+//   queue with one atomic per block per queue (block_append).
+// * tail: the last paths of a pass, each to its end in one launch (k_tail).
 // * film: per pixel, the samples of the pass are added in sample order into
 //   Kahan-compensated float sums of L and L^2: deterministic and reproducible.
 #include <algorithm>
@@ -137,9 +138,13 @@ __device__ __forceinline__ void block_append(const bool (&pred)[NQ], uint32_t* c
 
 // This file is compiled with fast single-precision division (reciprocal and multiply) and
 // flushes single-precision denormals; the two reciprocals of the traversal stay correctly
-// rounded: the double quotient of two floats rounded to float is the correctly rounded float
-// quotient (53 >= 2 * 24 + 2 bits make the double rounding innocuous).
-__device__ __forceinline__ float rcp_rn(float x) { return (float)(1.0 / (double)x); }
+// rounded: one Newton step on the hardware's reciprocal, and v_div_fixup for zeros, infinities and
+// NaN.  Compared with the rounded double quotient for all 2^32 inputs: equal everywhere, in 4
+// instructions instead of an IEEE division's ~12 with two mode switches.
+__device__ __forceinline__ float rcp_rn(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-x, y, 1.0f), y, y), x, 1.0f);
+}
 
 // ---- ray/triangle (triangle.cc:98-178 in float) -----------------------------------------
 __device__ __forceinline__ bool tri_hit(const float4* __restrict__ tris, uint32_t k, float3 o, float3 d, float tmax,
@@ -178,129 +183,169 @@ struct Counters {
     uint32_t nodes, tris;
 };
 
+// A wave leaves its interior-node loop once fewer than this many eighths of its busy lanes are in it:
+// the lanes that hold leaves or have finished their rays then get work, instead of waiting for the
+// wave's longest descent.  2 M closest hits, by eighths (0: wait for all): 0 351, 2 300, 3 288, 4 285, 5
+// 283, 6 289 us; 1080p x 32 frame 25.9, 23.5, 22.9, 22.7, 22.7, 22.8 ms; batch 15.5, 14.7, 14.6, 14.6, 14.9,
+// 15.2 ms.
+constexpr uint32_t kStayEighths = 4;
 
-// One 4-wide node (8 float4: lo.x, lo.y, lo.z, hi.x, hi.y, hi.z of the four children,
-// their links, pad): slab-tests the four boxes against [0, tbest] in FMA form (plane t =
-// p * (1/d) - o * (1/d), one fused multiply-add per plane), continues with the
-// nearest hit child and pushes the other hit children farthest first, so they pop in
-// near-to-far order.  Returns the next node or leaf link (kSent when the stack is empty).
-template <bool COUNT, class Push, class Pop>
-__device__ __forceinline__ int32_t visit4(const float4* __restrict__ nodes, int32_t node, float3 inv, float3 oinv,
-                                          float tbest, Push& push, Pop& pop, Counters& cnt) {
-    // 64-byte node: origin, scale and 8-bit child planes (decoded as fmaf(q, scale, origin),
-    // boxes rounded outwards at build time), then the four links
-    const float4* nd = nodes + 4 * node;
-    const float4 A = nd[0], B = nd[1], C = nd[2], lk = nd[3];
-    if (COUNT) cnt.nodes++;
-    const uint32_t qlx = __float_as_uint(B.z), qly = __float_as_uint(B.w), qlz = __float_as_uint(C.x);
-    const uint32_t qhx = __float_as_uint(C.y), qhy = __float_as_uint(C.z), qhz = __float_as_uint(C.w);
-    auto dq = [](uint32_t w, int c, float sc, float o) { return fmaf((float)((w >> (8 * c)) & 255u), sc, o); };
-    auto plane4 = [&](uint32_t w, float sc, float o) {
-        return make_float4(dq(w, 0, sc, o), dq(w, 1, sc, o), dq(w, 2, sc, o), dq(w, 3, sc, o));
-    };
-    const float4 lx = plane4(qlx, A.w, A.x), ly = plane4(qly, B.x, A.y), lz = plane4(qlz, B.y, A.z);
-    const float4 hx = plane4(qhx, A.w, A.x), hy = plane4(qhy, B.x, A.y), hz = plane4(qhz, B.y, A.z);
-    const float kNone = __int_as_float(0x7f800000);  // +inf: sorts after every hit
-    auto slab = [&](float ax, float ay, float az, float bx, float by, float bz, int32_t link) {
-        const float l_x = fmaf(ax, inv.x, -oinv.x), h_x = fmaf(bx, inv.x, -oinv.x);
-        const float l_y = fmaf(ay, inv.y, -oinv.y), h_y = fmaf(by, inv.y, -oinv.y);
-        const float l_z = fmaf(az, inv.z, -oinv.z), h_z = fmaf(bz, inv.z, -oinv.z);
-        const float tn = fmaxf(fmaxf(fminf(l_x, h_x), fminf(l_y, h_y)), fmaxf(fminf(l_z, h_z), 0.0f));
-        const float tf = fminf(fminf(fmaxf(l_x, h_x), fmaxf(l_y, h_y)), fminf(fmaxf(l_z, h_z), tbest));
-        return (tn <= tf * kRobust && link != kSent) ? tn : kNone;
-    };
-    int32_t c0 = __float_as_int(lk.x), c1 = __float_as_int(lk.y), c2 = __float_as_int(lk.z), c3 = __float_as_int(lk.w);
-    float k0 = slab(lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, c0);
-    float k1 = slab(lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, c1);
-    float k2 = slab(lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, c2);
-    float k3 = slab(lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, c3);
-    const int n = (k0 != kNone) + (k1 != kNone) + (k2 != kNone) + (k3 != kNone);
-    if (n == 0) return pop();
-    auto cx = [](float& ka, int32_t& ca, float& kb, int32_t& cb) {
-        const bool sw = kb < ka;
-        const float kt = sw ? kb : ka;
-        const int32_t ct = sw ? cb : ca;
-        kb = sw ? ka : kb;
-        cb = sw ? ca : cb;
-        ka = kt;
-        ca = ct;
-    };
-    // ascending by entry distance (misses last): a 5-comparator network
-    cx(k0, c0, k1, c1);
-    cx(k2, c2, k3, c3);
-    cx(k0, c0, k2, c2);
-    cx(k1, c1, k3, c3);
-    cx(k1, c1, k2, c2);
-    if (n > 3) push(c3);
-    if (n > 2) push(c2);
-    if (n > 1) push(c1);
-    return c0;
-}
+// One lane's walk down the BVH.  Every traversal kernel uses it: start() a ray, then step() (the
+// whole wave together) until done().
+//
+// Bound: VALU issue.  A node visit is ~150 VALU instructions and the closest-hit kernel keeps its
+// SIMDs' issue ports full, so what counts is instructions per visit and lanes per instruction, not
+// fetch latency (eight waves per SIMD cover it).  1080p x 32 frame, closest hits: 26 lanes of 64 active
+// per VALU instruction and 14.0 ms a pass while a wave stayed in its node loop until every lane held a
+// leaf; 38 lanes, a third fewer instructions and 10.1 ms now (the L1 tags are then 62% busy).
+// 2,000,003 closest hits 465 -> 264 us, 300,007 bounded any-hit rays 81 -> 57 us.
+//
+// The stack holds the S most recent entries in LDS (slot s at col[s * BLOCK], lanes on distinct
+// banks) and the rest in `spill`; its bottom entry is kSent, so a pop needs no empty check.
+template <int BLOCK, int S, bool COUNT>
+struct Walker {
+    float3 o, d, inv, oinv;
+    float tbest, hu, hv;
+    int32_t node, leaf, hit;  // node or leaf link in hand; postponed leaf link or 0; triangle or -1
+    int sp, spilled;
+    uint32_t* col;
+    uint32_t* spill;
 
-// Closest hit (ANY = false) or first hit (ANY = true).  Returns the leaf-order
-// triangle index or -1.  `col` is this lane's LDS stack column (slot s at
-// col[s * BLOCK]); `spill` holds entries below the S most recent ones.
-template <int BLOCK, int S, bool ANY, bool COUNT>
-__device__ __forceinline__ int32_t traverse(const SceneDev& sc, float3 o, float3 d, float tmax, float& t_out, float& u_out,
-                                            float& v_out, uint32_t* col, uint32_t* spill, bool active, Counters& cnt) {
-    const float4* __restrict__ nodes = sc.nodes;
-    const float4* __restrict__ tris = sc.tris;
-    float3 inv = safe_inv(d);
-    const float3 oinv = mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-    int32_t node = (active && sc.has_bvh) ? 0 : kSent;
-    int32_t leaf = 0;  // pending leaf link (negative) or 0
-    int sp = 0, spilled = 0;
-    int32_t hit = -1;
-    float tbest = tmax, hu = 0.0f, hv = 0.0f;
+    __device__ __forceinline__ void idle() {
+        o = d = inv = oinv = mk(0, 0, 0);
+        tbest = hu = hv = 0.0f;
+        node = kSent;
+        leaf = 0;
+        hit = -1;
+        sp = spilled = 0;
+    }
+    __device__ __forceinline__ void start(float3 org, float3 dir, float tmax, bool has_bvh) {
+        o = org;
+        d = dir;
+        inv = safe_inv(d);
+        oinv = mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+        tbest = tmax;
+        hu = hv = 0.0f;
+        node = has_bvh ? 0 : kSent;
+        leaf = 0;
+        hit = -1;
+        col[0] = (uint32_t)kSent;
+        sp = 1;
+        spilled = 0;
+    }
+    __device__ __forceinline__ bool done() const { return node == kSent && leaf == 0; }
 
-    auto push = [&](int32_t x) {
+    __device__ __forceinline__ void push(int32_t x) {
         if (sp - spilled == S) {
             spill[spilled] = col[(spilled & (S - 1)) * BLOCK];
             spilled++;
         }
         col[(sp & (S - 1)) * BLOCK] = (uint32_t)x;
         sp++;
-    };
-    auto pop = [&]() -> int32_t {
-        if (sp == 0) return kSent;
+    }
+    __device__ __forceinline__ int32_t pop() {
         sp--;
+        int32_t x = (int32_t)col[(sp & (S - 1)) * BLOCK];
         if (sp < spilled) {
             spilled = sp;
-            return (int32_t)spill[sp];
+            x = (int32_t)spill[sp];
         }
-        return (int32_t)col[(sp & (S - 1)) * BLOCK];
-    };
+        return x;
+    }
 
-    for (;;) {
-        // Interior nodes until every lane of the wave holds a leaf (or is done).
+    // One 64-byte node: origin, scale and 8-bit planes of the four child boxes (decoded as
+    // fmaf(q, scale, origin), rounded outwards at build time), then the four links.  Slab tests in FMA
+    // form (plane t = p * (1/d) - o * (1/d)); the sign of the direction says which plane is the near
+    // one.  (Folding the decoding into the slab test, q (scale inv) + (origin inv - o inv), saves 18 of
+    // the visit's multiply-adds and 2-3% of the time, but its rounding lost and gained hits at box
+    // edges: 10 of 3e9 rays answered differently, against 2 with this form.)  Continues with the
+    // nearest hit child and pushes the others farthest first, so they pop in near-to-far order.
+    __device__ __forceinline__ void visit(const float4* __restrict__ nodes, Counters& cnt) {
+        const float4* nd = nodes + 4 * node;
+        const float4 A = nd[0], B = nd[1], C = nd[2], lk = nd[3];
+        if (COUNT) cnt.nodes++;
+        const uint32_t qlx = __float_as_uint(B.z), qly = __float_as_uint(B.w), qlz = __float_as_uint(C.x);
+        const uint32_t qhx = __float_as_uint(C.y), qhy = __float_as_uint(C.z), qhz = __float_as_uint(C.w);
+        const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
+        const uint32_t nx = sx ? qhx : qlx, ny = sy ? qhy : qly, nz = sz ? qhz : qlz;
+        const uint32_t fx = sx ? qlx : qhx, fy = sy ? qly : qhy, fz = sz ? qlz : qhz;
+        const float kNone = __int_as_float(0x7f800000);  // +inf: sorts after every hit
+        auto slab = [&](int c, int32_t link) {
+            auto at = [c](uint32_t w, float sc, float org, float i, float oi) {
+                return fmaf(fmaf((float)((w >> (8 * c)) & 255u), sc, org), i, -oi);
+            };
+            const float tn = fmaxf(fmaxf(at(nx, A.w, A.x, inv.x, oinv.x), at(ny, B.x, A.y, inv.y, oinv.y)),
+                                   fmaxf(at(nz, B.y, A.z, inv.z, oinv.z), 0.0f));
+            const float tf = fminf(fminf(at(fx, A.w, A.x, inv.x, oinv.x), at(fy, B.x, A.y, inv.y, oinv.y)),
+                                   fminf(at(fz, B.y, A.z, inv.z, oinv.z), tbest));
+            return (tn <= tf * kRobust && link != kSent) ? tn : kNone;
+        };
+        int32_t c0 = __float_as_int(lk.x), c1 = __float_as_int(lk.y), c2 = __float_as_int(lk.z),
+                c3 = __float_as_int(lk.w);
+        float k0 = slab(0, c0), k1 = slab(1, c1), k2 = slab(2, c2), k3 = slab(3, c3);
+        auto cx = [](float& ka, int32_t& ca, float& kb, int32_t& cb) {
+            const bool sw = kb < ka;
+            const float kt = sw ? kb : ka;
+            const int32_t ct = sw ? cb : ca;
+            kb = sw ? ka : kb;
+            cb = sw ? ca : cb;
+            ka = kt;
+            ca = ct;
+        };
+        // ascending by entry distance (misses last): a 5-comparator network
+        cx(k0, c0, k1, c1);
+        cx(k2, c2, k3, c3);
+        cx(k0, c0, k2, c2);
+        cx(k1, c1, k3, c3);
+        cx(k1, c1, k2, c2);
+        if (sp - spilled <= S - 3) {
+            // room for three: every slot is written, the count moves past those that hold a hit
+            col[(sp & (S - 1)) * BLOCK] = (uint32_t)c3;
+            sp += k3 != kNone ? 1 : 0;
+            col[(sp & (S - 1)) * BLOCK] = (uint32_t)c2;
+            sp += k2 != kNone ? 1 : 0;
+            col[(sp & (S - 1)) * BLOCK] = (uint32_t)c1;
+            sp += k1 != kNone ? 1 : 0;
+        } else {
+            if (k3 != kNone) push(c3);
+            if (k2 != kNone) push(c2);
+            if (k1 != kNone) push(c1);
+        }
+        if (k0 != kNone) node = c0;
+        else node = pop();
+    }
+
+    // Interior nodes until few of the wave's `busy` lanes have any left to visit, then the leaves in
+    // hand.  A lane holds one postponed leaf while it looks for the next, so a ray's triangles are
+    // tested in its own depth-first order whatever the other lanes do.
+    __device__ __forceinline__ void step(const float4* __restrict__ nodes, const float4* __restrict__ tris, bool any,
+                                         uint32_t busy, Counters& cnt) {
         while (node >= 0 && node != kSent) {
-            node = visit4<COUNT>(nodes, node, inv, oinv, tbest, push, pop, cnt);
+            visit(nodes, cnt);
             if (node < 0 && leaf == 0) {
                 leaf = node;
                 node = pop();
             }
             if (__all(leaf != 0)) break;
+            if ((uint32_t)__popcll(__ballot(1)) * 8u < busy * kStayEighths) break;
         }
-        // Leaves.
         while (leaf < 0) {
-            uint32_t x = ~(uint32_t)leaf;
-            uint32_t first = x >> kLeafCountBits, n = (x & (kMaxLeafTris - 1)) + 1;
+            const uint32_t x = ~(uint32_t)leaf;
+            const uint32_t first = x >> kLeafCountBits, n = (x & (kMaxLeafTris - 1)) + 1;
             for (uint32_t k = first; k < first + n; k++) {
                 float t, u, v;
                 if (COUNT) cnt.tris++;
                 if (tri_hit(tris, k, o, d, tbest, t, u, v)) {
                     hit = (int32_t)k;
-                    if (ANY) break;
+                    if (any) break;
                     tbest = t;
                     hu = u;
                     hv = v;
                 }
             }
-            if (ANY && hit >= 0) {
+            if (any && hit >= 0) {
                 node = kSent;
                 leaf = 0;
-                sp = 0;
-                spilled = 0;
                 break;
             }
             leaf = 0;
@@ -309,33 +354,29 @@ __device__ __forceinline__ int32_t traverse(const SceneDev& sc, float3 o, float3
                 node = pop();
             }
         }
-        if (node == kSent && leaf == 0) break;
     }
-    t_out = tbest;
-    u_out = hu;
-    v_out = hv;
-    return hit;
-}
+};
 
 // Static work split for the persistent traversal grids.  The hardware deals
 // workgroups round-robin over the 8 XCDs; renumbering so that XCD x owns the
 // logical blocks [x * G/8, (x+1) * G/8) gives each XCD (and its L2) a contiguous
 // slice of the queue, i.e. neighbouring, coherent rays.  Each wave then takes
-// 64-item chunks grid-stride: no shared counter, no atomics.
+// chunks of 2^chunk_log2 items grid-stride (64, or fewer where few rays are spread over many
+// waves): no shared counter, no atomics.
 constexpr uint32_t kXcds = 8;
 struct WaveSplit {
     uint32_t first;   // first item of this wave
     uint32_t stride;  // items between successive chunks of this wave
 };
 template <int BLOCK>
-__device__ __forceinline__ WaveSplit wave_split() {
+__device__ __forceinline__ WaveSplit wave_split(uint32_t chunk_log2) {
     uint32_t g = gridDim.x, b = blockIdx.x;
     uint32_t logical = b;
     if (g % kXcds == 0) logical = (b % kXcds) * (g / kXcds) + b / kXcds;
     uint32_t wave = logical * (BLOCK / 64) + threadIdx.x / 64;
     WaveSplit s;
-    s.first = wave * 64u;
-    s.stride = g * (uint32_t)BLOCK;
+    s.first = wave << chunk_log2;
+    s.stride = (g * (uint32_t)(BLOCK / 64)) << chunk_log2;
     return s;
 }
 
@@ -346,10 +387,7 @@ __device__ __forceinline__ WaveSplit wave_split() {
 // load(i, o, d, tmax) reads ray i and returns its scene (batch: an entry of the scene
 // table; single: null, the kernel's scene argument is used); done(i, hit, t, u, v, scene)
 // consumes its result.
-#ifndef SPK_REFILL
-#define SPK_REFILL 8
-#endif
-constexpr int kRefill = SPK_REFILL;
+constexpr int kRefill = 8;
 
 template <bool BATCH>
 __device__ __forceinline__ const SceneDev& pick_scene(const SceneDev* p, const SceneDev& s) {
@@ -359,108 +397,47 @@ __device__ __forceinline__ const SceneDev& pick_scene(const SceneDev* p, const S
 
 template <int BLOCK, int S, bool ANY, bool COUNT, bool BATCH, class Load, class Done>
 __device__ __forceinline__ void traverse_stream(const SceneDev& sc0, const SceneDev* scenes, uint32_t count, Load load,
-                                                Done done, uint32_t* col, uint32_t* spill, Counters& cnt) {
-    const WaveSplit ws = wave_split<BLOCK>();
+                                                Done done, uint32_t* col, uint32_t* spill, Counters& cnt,
+                                                uint32_t chunk_log2 = 6) {
+    const WaveSplit ws = wave_split<BLOCK>(chunk_log2);
+    const uint32_t lanes = 1u << chunk_log2;  // rays a wave holds at a time
+    const bool usable = (uint32_t)__lane_id() < lanes;
     bool active = false;
     uint32_t idx = 0;
     const SceneDev* sc = scenes;  // batch only: this lane's scene
-    float3 o = mk(0, 0, 0), d = mk(0, 0, 1), inv = mk(1, 1, 1), oinv = mk(0, 0, 0);
-    int32_t node = kSent, leaf = 0;
-    int sp = 0, spilled = 0;
-    int32_t hit = -1;
-    float tbest = 0.0f, hu = 0.0f, hv = 0.0f;
+    Walker<BLOCK, S, COUNT> w;
+    w.idle();
+    w.col = col;
+    w.spill = spill;
     uint32_t cursor = 0;  // wave-uniform: positions of the wave's slice handed out so far
-    auto index_of = [&](uint32_t pos) { return ws.first + (pos >> 6) * ws.stride + (pos & 63u); };
+    auto index_of = [&](uint32_t pos) { return ws.first + (pos >> chunk_log2) * ws.stride + (pos & (lanes - 1u)); };
     bool exhausted = index_of(0) >= count;
-
-    auto push = [&](int32_t x) {
-        if (sp - spilled == S) {
-            spill[spilled] = col[(spilled & (S - 1)) * BLOCK];
-            spilled++;
-        }
-        col[(sp & (S - 1)) * BLOCK] = (uint32_t)x;
-        sp++;
-    };
-    auto pop = [&]() -> int32_t {
-        if (sp == 0) return kSent;
-        sp--;
-        if (sp < spilled) {
-            spilled = sp;
-            return (int32_t)spill[sp];
-        }
-        return (int32_t)col[(sp & (S - 1)) * BLOCK];
-    };
-
     for (;;) {
         if (!exhausted) {
-            const uint64_t idle = __ballot(!active);
+            const uint64_t idle = __ballot(usable && !active);
             const uint32_t n_idle = (uint32_t)__popcll(idle);
-            if (n_idle >= (uint32_t)kRefill || n_idle == 64u) {
-                if (!active) {
+            if (n_idle >= (uint32_t)kRefill || n_idle == lanes) {
+                if (usable && !active) {
                     const uint32_t i = index_of(cursor + (uint32_t)__popcll(idle & ((1ull << __lane_id()) - 1ull)));
                     if (i < count) {
+                        float3 o, d;
                         float tmax;
                         const SceneDev* ls = load(i, o, d, tmax);
                         if constexpr (BATCH) sc = ls;
                         idx = i;
                         active = true;
-                        inv = safe_inv(d);
-                        oinv = mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-                        node = pick_scene<BATCH>(sc, sc0).has_bvh ? 0 : kSent;
-                        leaf = 0;
-                        sp = 0;
-                        spilled = 0;
-                        hit = -1;
-                        tbest = tmax;
-                        hu = hv = 0.0f;
+                        w.start(o, d, tmax, pick_scene<BATCH>(sc, sc0).has_bvh != 0);
                     }
                 }
                 cursor += n_idle;
                 exhausted = index_of(cursor) >= count;
             }
         }
-        if (!__any(active)) break;
-        const float4* __restrict__ nodes = pick_scene<BATCH>(sc, sc0).nodes;
-        const float4* __restrict__ tris = pick_scene<BATCH>(sc, sc0).tris;
-        // Interior nodes until every busy lane holds a leaf (or is done).
-        while (node >= 0 && node != kSent) {
-            node = visit4<COUNT>(nodes, node, inv, oinv, tbest, push, pop, cnt);
-            if (node < 0 && leaf == 0) {
-                leaf = node;
-                node = pop();
-            }
-            if (__all(leaf != 0)) break;
-        }
-        // Leaves.
-        while (leaf < 0) {
-            uint32_t x = ~(uint32_t)leaf;
-            uint32_t first = x >> kLeafCountBits, n = (x & (kMaxLeafTris - 1)) + 1;
-            for (uint32_t k = first; k < first + n; k++) {
-                float t, u, v;
-                if (COUNT) cnt.tris++;
-                if (tri_hit(tris, k, o, d, tbest, t, u, v)) {
-                    hit = (int32_t)k;
-                    if (ANY) break;
-                    tbest = t;
-                    hu = u;
-                    hv = v;
-                }
-            }
-            if (ANY && hit >= 0) {
-                node = kSent;
-                leaf = 0;
-                sp = 0;
-                spilled = 0;
-                break;
-            }
-            leaf = 0;
-            if (node < 0) {
-                leaf = node;
-                node = pop();
-            }
-        }
-        if (active && node == kSent && leaf == 0) {
-            done(idx, hit, tbest, hu, hv, pick_scene<BATCH>(sc, sc0));
+        const uint32_t busy = (uint32_t)__popcll(__ballot(active));
+        if (busy == 0) break;
+        w.step(pick_scene<BATCH>(sc, sc0).nodes, pick_scene<BATCH>(sc, sc0).tris, ANY, busy, cnt);
+        if (active && w.done()) {
+            done(idx, w.hit, w.tbest, w.hu, w.hv, pick_scene<BATCH>(sc, sc0));
             active = false;
         }
     }
@@ -468,35 +445,29 @@ __device__ __forceinline__ void traverse_stream(const SceneDev& sc0, const Scene
 
 // ---- standalone trace (spk_trace) --------------------------------------------------------
 template <int BLOCK, int S, bool ANY>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_trace(SceneDev sc, TraceBufs b, uint32_t* work, uint32_t* spill_all,
-                                                 int spill_cap) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_trace(SceneDev sc, TraceBufs b,
+                                                                                        uint32_t* spill_all, int spill_cap,
+                                                                                        uint32_t chunk_log2) {
     __shared__ uint32_t lds[S * BLOCK];
     uint32_t* col = lds + threadIdx.x;
     uint32_t* spill = spill_all + (size_t)(blockIdx.x * BLOCK + threadIdx.x) * spill_cap;
-    const uint64_t n = (uint64_t)b.n;
-    const WaveSplit ws = wave_split<BLOCK>();
-    for (uint64_t base = ws.first; base < n; base += ws.stride) {
-        uint64_t i = base + __lane_id();
-        bool active = i < n;
-        float3 o = mk(0, 0, 1), d = mk(0, 0, 1);
-        float tmax = kINFTY;
-        if (active) {
-            o = mk(b.org[3 * i], b.org[3 * i + 1], b.org[3 * i + 2]);
-            d = normalize(mk(b.dir[3 * i], b.dir[3 * i + 1], b.dir[3 * i + 2]));
-            if (b.tmax) tmax = b.tmax[i];
+    Counters cnt = {0, 0};
+    auto load = [&](uint32_t j, float3& o, float3& d, float& tmax) -> const SceneDev* {
+        const size_t i = j;
+        o = mk(b.org[3 * i], b.org[3 * i + 1], b.org[3 * i + 2]);
+        d = normalize(mk(b.dir[3 * i], b.dir[3 * i + 1], b.dir[3 * i + 2]));
+        tmax = b.tmax ? b.tmax[i] : kINFTY;
+        return nullptr;
+    };
+    auto done = [&](uint32_t i, int32_t k, float t, float, float, const SceneDev& s) {
+        if (ANY) {
+            b.prim_out[i] = k >= 0 ? 1 : 0;
+        } else {
+            b.prim_out[i] = k >= 0 ? s.tri_ids[k].x : -1;
+            if (b.t_out) b.t_out[i] = k >= 0 ? t : -1.0f;
         }
-        float t, u, v;
-        Counters cnt = {0, 0};
-        int32_t k = traverse<BLOCK, S, ANY, false>(sc, o, d, tmax, t, u, v, col, spill, active, cnt);
-        if (active) {
-            if (ANY) {
-                b.prim_out[i] = k >= 0 ? 1 : 0;
-            } else {
-                b.prim_out[i] = k >= 0 ? sc.tri_ids[k].x : -1;
-                if (b.t_out) b.t_out[i] = k >= 0 ? t : -1.0f;
-            }
-        }
-    }
+    };
+    traverse_stream<BLOCK, S, ANY, false, false>(sc, nullptr, (uint32_t)b.n, load, done, col, spill, cnt, chunk_log2);
 }
 
 // ---- pass bookkeeping -----------------------------------------------------------------------
@@ -1942,98 +1913,35 @@ template <int BLOCK, int S>
 __device__ __forceinline__ void traverse_pair(const SceneDev& sc, bool has1, bool any1, float3 o, float3 d, float tmax,
                                               bool has2, float3 o2, float3 d2, float4& hit1, int32_t& hit2, uint32_t* col,
                                               uint32_t* spill) {
-    const float4* __restrict__ nodes = sc.nodes;
-    const float4* __restrict__ tris = sc.tris;
-    const int32_t root = sc.has_bvh ? 0 : kSent;
+    const bool bvh = sc.has_bvh != 0;
     Counters cnt = {0, 0};
-    float3 inv = mk(1, 1, 1), oinv = mk(0, 0, 0);
-    int32_t node = kSent, leaf = 0, hit = -1;
-    int sp = 0, spilled = 0;
-    float tbest = 0.0f, hu = 0.0f, hv = 0.0f;
+    Walker<BLOCK, S, false> w;
+    w.idle();
+    w.col = col;
+    w.spill = spill;
     bool any = false;
     int ray = 0;  // the ray in flight: 1, 2, or 0 for none
-    auto push = [&](int32_t x) {
-        if (sp - spilled == S) {
-            spill[spilled] = col[(spilled & (S - 1)) * BLOCK];
-            spilled++;
-        }
-        col[(sp & (S - 1)) * BLOCK] = (uint32_t)x;
-        sp++;
-    };
-    auto pop = [&]() -> int32_t {
-        if (sp == 0) return kSent;
-        sp--;
-        if (sp < spilled) {
-            spilled = sp;
-            return (int32_t)spill[sp];
-        }
-        return (int32_t)col[(sp & (S - 1)) * BLOCK];
-    };
     hit1 = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(-1));
     hit2 = -1;
     for (;;) {
-        if (ray == 0 && (has1 || has2)) {
-            if (has1) {
-                ray = 1;
-                any = any1;
-                tbest = tmax;
-            } else {
-                ray = 2;
-                any = false;
-                tbest = kINFTY;
-                o = o2;
-                d = d2;
-            }
-            inv = safe_inv(d);
-            oinv = mk(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-            node = root;
-            leaf = 0;
-            sp = 0;
-            spilled = 0;
-            hit = -1;
-            hu = hv = 0.0f;
+        if (ray == 0 && has1) {
+            ray = 1;
+            any = any1;
+            w.start(o, d, tmax, bvh);
+        } else if (ray == 0 && has2) {
+            ray = 2;
+            any = false;
+            w.start(o2, d2, kINFTY, bvh);
         }
-        if (!__any(ray != 0)) break;
-        while (node >= 0 && node != kSent) {
-            node = visit4<false>(nodes, node, inv, oinv, tbest, push, pop, cnt);
-            if (node < 0 && leaf == 0) {
-                leaf = node;
-                node = pop();
-            }
-            if (__all(leaf != 0)) break;
-        }
-        while (leaf < 0) {
-            uint32_t x = ~(uint32_t)leaf;
-            uint32_t first = x >> kLeafCountBits, n = (x & (kMaxLeafTris - 1)) + 1;
-            for (uint32_t k = first; k < first + n; k++) {
-                float t, u, v;
-                if (tri_hit(tris, k, o, d, tbest, t, u, v)) {
-                    hit = (int32_t)k;
-                    if (any) break;
-                    tbest = t;
-                    hu = u;
-                    hv = v;
-                }
-            }
-            if (any && hit >= 0) {
-                node = kSent;
-                leaf = 0;
-                sp = 0;
-                spilled = 0;
-                break;
-            }
-            leaf = 0;
-            if (node < 0) {
-                leaf = node;
-                node = pop();
-            }
-        }
-        if (ray != 0 && node == kSent && leaf == 0) {
+        const uint32_t busy = (uint32_t)__popcll(__ballot(ray != 0));
+        if (busy == 0) break;
+        w.step(sc.nodes, sc.tris, any, busy, cnt);
+        if (ray != 0 && w.done()) {
             if (ray == 1) {
-                hit1 = make_float4(tbest, hu, hv, __int_as_float(hit));
+                hit1 = make_float4(w.tbest, w.hu, w.hv, __int_as_float(w.hit));
                 has1 = false;
             } else {
-                hit2 = hit;
+                hit2 = w.hit;
                 has2 = false;
             }
             ray = 0;
@@ -2545,13 +2453,35 @@ int trace_blocks_per_cu(int block) {
 int tail_waves_per_cu() { return kTailWavesPerCu; }
 
 // ---- launchers ---------------------------------------------------------------------------------------
-int launch_trace(const SceneDev& s, const TraceBufs& b, uint32_t* work_counter, uint32_t* spill, int spill_cap, int grid,
-                 hipStream_t st) {
+// Rays in pieces a 32-bit index strides over without wrapping; no more blocks than hold rays.
+int launch_trace(const SceneDev& s, const TraceBufs& b, uint32_t* spill, int spill_cap, int grid, hipStream_t st) {
     constexpr int B = 128;
-    if (b.any_hit)
-        hipLaunchKernelGGL((k_trace<B, kStackSlots, true>), dim3(grid), dim3(B), 0, st, s, b, work_counter, spill, spill_cap);
-    else
-        hipLaunchKernelGGL((k_trace<B, kStackSlots, false>), dim3(grid), dim3(B), 0, st, s, b, work_counter, spill, spill_cap);
+    constexpr int64_t kPiece = int64_t(1) << 30;
+    constexpr int64_t kSpreadWaves = 4096;
+    for (int64_t i0 = 0; i0 < b.n; i0 += kPiece) {
+        TraceBufs p = b;
+        p.n = std::min(kPiece, b.n - i0);
+        p.org += 3 * i0;
+        p.dir += 3 * i0;
+        if (p.tmax) p.tmax += i0;
+        p.prim_out += i0;
+        if (p.t_out) p.t_out += i0;
+        // Few rays: fewer lanes per wave, up to kSpreadWaves waves, so that a wave waits for fewer
+        // rays (us a call, 64 rays a wave / this rule: 257 rays 14.6 / 11.4, 3,000 52 / 40, 10,000 40 /
+        // 35, 30,000 46 / 41, 60,000 78 / 69; at 100,000 the sizes are level and below 64 lanes lose).
+        uint32_t c = 0;
+        while (c < 6 && (p.n >> c) > kSpreadWaves) c++;
+        if (c == 5) c = 6;
+        // Many rays: every wave the same number of chunks, for no wave should start another when the
+        // rest is done (700,000 rays 183 -> 132 us, 2,000,003 291 -> 264), and two from where the chip is
+        // still a third full, so that finished lanes have a ray to go on with (300,007 any-hit 61 -> 57).
+        const int64_t block_chunk = (int64_t)(B / 64) << c;
+        int64_t m = (p.n + grid * block_chunk - 1) / (grid * block_chunk);
+        if (m == 1 && p.n * 3 > grid * block_chunk && c == 6) m = 2;
+        const int g = (int)std::min<int64_t>(grid, (p.n + m * block_chunk - 1) / (m * block_chunk));
+        if (b.any_hit) hipLaunchKernelGGL((k_trace<B, kStackSlots, true>), dim3(g), dim3(B), 0, st, s, p, spill, spill_cap, c);
+        else hipLaunchKernelGGL((k_trace<B, kStackSlots, false>), dim3(g), dim3(B), 0, st, s, p, spill, spill_cap, c);
+    }
     SPK_CHECK_HIP(hipGetLastError());
     return SPK_OK;
 }

@@ -3,16 +3,16 @@
 // serving loops, harnesses that forbid allocation).
 //
 // spk_trace allocates its traversal scratch lazily per scene: a per-thread overflow area for
-// the traversal stack (entries past the LDS slots) and a work word.  Here that scratch is one
+// the traversal stack (entries past the LDS slots).  Here that scratch is one
 // file-scope device array, `scratch`, of kNoAllocScratchBytes per GPU, which every GPU holds
 // from the library's load until the process ends.  Its device address is looked up once per
 // device with hipGetSymbolAddress and only that address is handed to kernels.  The kernels
-// and results are spk_trace's: rays are assigned to waves in fixed 64-ray chunks whatever the
-// grid, so a grid shrunk to fit the scratch traces every ray exactly as spk_trace does.
+// and results are spk_trace's: a ray's own visiting order does not depend on the grid, so a grid
+// shrunk to fit the scratch traces every ray as spk_trace does.
 //
 // Nothing in the scratch needs clearing between calls: a thread writes a spill slot before it
-// reads it, and the work word is not read by the trace kernel.  All calls on one GPU share the
-// array, so calls that overlap on one GPU (two streams, two host threads) race on it.
+// reads it.  All calls on one GPU share the array, so calls that overlap on one GPU (two streams,
+// two host threads) race on it.
 #include <algorithm>
 #include <mutex>
 
@@ -22,7 +22,7 @@ namespace spk {
 namespace {
 
 constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;  // 32 MiB per GPU
-constexpr size_t kNoAllocWorkBytes = 256;                   // the work word, padded
+constexpr size_t kNoAllocHeadBytes = 256;                   // not used by the stacks
 constexpr int kNoAllocBlock = 128;                          // launch_trace's block size
 constexpr int kMaxDevices = 64;
 
@@ -80,11 +80,11 @@ extern "C" int spk_trace_noalloc(spk_scene* s, const float* org, const float* di
     scene_trace_info(s, &si);
     // each persistent thread owns spill_cap stack words; a block of them must fit
     const size_t per_block = (size_t)kNoAllocBlock * (size_t)si.spill_cap * 4u;
-    const size_t max_blocks = (kNoAllocScratchBytes - kNoAllocWorkBytes) / per_block;
+    const size_t max_blocks = (kNoAllocScratchBytes - kNoAllocHeadBytes) / per_block;
     if (max_blocks < 1) {
         set_error("spk_trace_noalloc: the scene's BVH needs %zu bytes of stack overflow per block, more than the "
                   "%zu-byte scratch holds",
-                  per_block, kNoAllocScratchBytes - kNoAllocWorkBytes);
+                  per_block, kNoAllocScratchBytes - kNoAllocHeadBytes);
         return SPK_ERR_INVALID;
     }
     if (n == 0) return SPK_OK;
@@ -101,7 +101,6 @@ extern "C" int spk_trace_noalloc(spk_scene* s, const float* org, const float* di
     b.t_out = t_out;
     b.n = n;
     b.any_hit = any_hit ? 1 : 0;
-    uint32_t* work = reinterpret_cast<uint32_t*>(ds.ptr);
-    uint32_t* spill = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(ds.ptr) + kNoAllocWorkBytes);
-    return launch_trace(*si.dev, b, work, spill, si.spill_cap, grid, (hipStream_t)stream);
+    uint32_t* spill = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(ds.ptr) + kNoAllocHeadBytes);
+    return launch_trace(*si.dev, b, spill, si.spill_cap, grid, (hipStream_t)stream);
 }
