@@ -31,13 +31,20 @@ constexpr float kGLogKappaLo = -4.0f, kGLogKappaHi = 7.0f;
 // Flat parameter vector (logical order): W1[64][224] b1 W2[64][64] b2 W3 b3 W4 b4 W5[40][64] b5.
 constexpr int kGOffW1 = 0, kGOffB1 = 14336, kGOffW2 = 14400, kGOffB2 = 18496, kGOffW3 = 18560, kGOffB3 = 22656,
               kGOffW4 = 22720, kGOffB4 = 26816, kGOffW5 = 26880, kGOffB5 = 29440, kGParams = 29480;
-// Forward bf16 image: W1 [64][224] natural, W2..W4 [64][64] and W5 [48][64] in slot order.
-constexpr int kGFwdW1 = 0, kGFwdW2 = 14336, kGFwdW3 = 18432, kGFwdW4 = 22528, kGFwdW5 = 26624, kGFwdSize = 29696;
+// The bf16 images are copied into LDS as they are and read there as MFMA A operands, 16 bytes a lane:
+// lane r of 16 reads row r.  Rows are padded by 8, so that the lanes of a read meet the banks evenly.
+constexpr int kGRow1 = kGEnc + 8;
+constexpr int kGRowH = kGHid + 8;
+// Forward bf16 image: W1 [64][kGRow1] natural, W2..W4 [64][kGRowH] and W5 [48][kGRowH] in slot order.
+constexpr int kGFwdW1 = 0, kGFwdW2 = 64 * kGRow1, kGFwdW3 = kGFwdW2 + 64 * kGRowH, kGFwdW4 = kGFwdW3 + 64 * kGRowH,
+              kGFwdW5 = kGFwdW4 + 64 * kGRowH, kGFwdSize = kGFwdW5 + 48 * kGRowH;
 // Biases in fp32: b1..b4 at 64 l, b5 at 256 (48 with zero padding).
 constexpr int kGBiasSize = 304;
-// Backward bf16 image: WT2..WT4 [64][64] (rows = input unit, K in slot order of the
-// layer's outputs) and WT5 [64][64] (K = output index 0..39, zero padded).
-constexpr int kGBwdWT2 = 0, kGBwdWT3 = 4096, kGBwdWT4 = 8192, kGBwdWT5 = 12288, kGBwdSize = 16384;
+// Backward bf16 image: WT2..WT4 [64][kGRowH] (rows = input unit, K in slot order of the
+// layer's outputs) and WT5 [64][kGRowH] (K = output index 0..39, zero padded).
+constexpr int kGBwdWT2 = 0, kGBwdWT3 = 64 * kGRowH, kGBwdWT4 = 128 * kGRowH, kGBwdWT5 = 192 * kGRowH,
+              kGBwdSize = 256 * kGRowH;
+static_assert(kGFwdSize % 8 == 0 && kGBwdSize % 8 == 0, "images are copied 16 bytes at a time");
 
 __host__ __device__ constexpr int slot_unit(int s) {
     return 16 * (2 * (s >> 5) + ((s & 7) >> 2)) + 4 * ((s >> 3) & 3) + (s & 3);
@@ -163,7 +170,7 @@ __device__ __forceinline__ void mlp_forward(const uint16_t* __restrict__ w, cons
         }
 #pragma unroll
         for (int mt = 0; mt < 4; mt++) {
-            const u32x4_t a = ld16(w + kGFwdW1 + (16 * mt + r) * kGEnc + 32 * c + 8 * g);
+            const u32x4_t a = ld16(w + kGFwdW1 + (16 * mt + r) * kGRow1 + 32 * c + 8 * g);
 #pragma unroll
             for (int ct = 0; ct < NCT; ct++) acc[mt][ct] = mfma_bf16(a, b[ct], acc[mt][ct]);
         }
@@ -179,7 +186,7 @@ __device__ __forceinline__ void mlp_forward(const uint16_t* __restrict__ w, cons
         for (int c = 0; c < 2; c++)
 #pragma unroll
             for (int mt = 0; mt < 4; mt++) {
-                const u32x4_t a = ld16(w + offs[l] + (16 * mt + r) * kGHid + 32 * c + 8 * g);
+                const u32x4_t a = ld16(w + offs[l] + (16 * mt + r) * kGRowH + 32 * c + 8 * g);
 #pragma unroll
                 for (int ct = 0; ct < NCT; ct++) acc[mt][ct] = mfma_bf16(a, h[c][ct], acc[mt][ct]);
             }
@@ -191,7 +198,7 @@ __device__ __forceinline__ void mlp_forward(const uint16_t* __restrict__ w, cons
     for (int c = 0; c < 2; c++)
 #pragma unroll
         for (int mt = 0; mt < 3; mt++) {
-            const u32x4_t a = ld16(w + kGFwdW5 + (16 * mt + r) * kGHid + 32 * c + 8 * g);
+            const u32x4_t a = ld16(w + kGFwdW5 + (16 * mt + r) * kGRowH + 32 * c + 8 * g);
 #pragma unroll
             for (int ct = 0; ct < NCT; ct++) out[mt][ct] = mfma_bf16(a, h[c][ct], out[mt][ct]);
         }

@@ -36,7 +36,7 @@ constexpr float kGuideClip = SPK_GUIDE_CLIP;
 __device__ void write_param_images(int p, float th, uint16_t* wf, uint16_t* wb, float* bias) {
     const uint16_t h = (uint16_t)bf16_bits(th);
     if (p < kGOffB1) {
-        wf[kGFwdW1 + p] = h;
+        wf[kGFwdW1 + (p / kGEnc) * kGRow1 + p % kGEnc] = h;
         return;
     }
     if (p < kGOffW2) {
@@ -49,8 +49,8 @@ __device__ void write_param_images(int p, float th, uint16_t* wf, uint16_t* wb, 
     }
     if (p >= kGOffW5) {
         const int q = p - kGOffW5, n = q >> 6, k = q & 63;
-        wf[kGFwdW5 + n * 64 + unit_slot(k)] = h;
-        wb[kGBwdWT5 + k * 64 + n] = h;
+        wf[kGFwdW5 + n * kGRowH + unit_slot(k)] = h;
+        wb[kGBwdWT5 + k * kGRowH + n] = h;
         return;
     }
     // layers 2..4: blocks of 4096 weights + 64 biases
@@ -60,8 +60,8 @@ __device__ void write_param_images(int p, float th, uint16_t* wf, uint16_t* wb, 
         return;
     }
     const int n = o >> 6, k = o & 63;
-    wf[kGFwdW2 + 4096 * l + n * 64 + unit_slot(k)] = h;
-    wb[kGBwdWT2 + 4096 * l + k * 64 + unit_slot(n)] = h;
+    wf[kGFwdW2 + 64 * kGRowH * l + n * kGRowH + unit_slot(k)] = h;
+    wb[kGBwdWT2 + 64 * kGRowH * l + k * kGRowH + unit_slot(n)] = h;
 }
 
 __global__ void k_guide_images(const float* __restrict__ params, uint16_t* wf, uint16_t* wb, float* bias) {
@@ -154,8 +154,6 @@ __global__ void k_guide_step_begin(GuideState* gs, uint32_t batch, uint32_t rec_
     pcg4d(h0, h1, h2, h3);
     gs->perm_a = a;
     gs->perm_off = n > 0 ? h0 % n : 0u;
-    gs->loss_sum = 0.0f;
-    gs->weight_sum = 0.0f;
     // the last training step's gradient norm joins the running mean (clipped as it was)
     if (gs->gnorm2 > 0.0f) {
         const float norm = sqrtf(gs->gnorm2), ema = gs->gnorm_ema;
@@ -240,13 +238,19 @@ __device__ __forceinline__ void mask_pack(const f32x4_t (&d)[4], const u32x4_t (
 }
 
 // Persistent blocks (one per CU): the forward and backward weight images are staged in
-// LDS once, then each wave takes 16-sample tiles.
-__global__ __launch_bounds__(256) void k_guide_fb(const uint16_t* __restrict__ wf, const float* __restrict__ bias,
-                                                  const uint16_t* __restrict__ wb, TrainBufs tb, GuideState* gs) {
+// LDS once, then each wave takes 16-sample tiles.  Bound: the 1,152 bytes of activations and deltas it
+// writes a sample (302 MB for 2^18, 3.5 TB/s; without the writes 30 us less).  The four lanes that share a
+// sample take two lobes of the loss each (sums over lobes are still formed lobe by lobe, in every lane
+// alike).  2^18 samples 150 -> 87 us, 2^14 42 -> 19 us.
+constexpr int kFbWaves = 16;  // at most (128 VGPRs, 144 KB of LDS); the launch takes as many as it has tiles for
+__global__ __launch_bounds__(64 * kFbWaves) void k_guide_fb(const uint16_t* __restrict__ wf, const float* __restrict__ bias,
+                                                           const uint16_t* __restrict__ wb, TrainBufs tb,
+                                                           const GuideState* __restrict__ gs, float2* loss_part) {
     __shared__ __attribute__((aligned(16))) uint16_t wf_lds[kGFwdSize];
     __shared__ __attribute__((aligned(16))) uint16_t wb_lds[kGBwdSize];
     __shared__ float b_lds[kGBiasSize];
-    __shared__ float dl[4][16 * 41];
+    __shared__ float dl[kFbWaves][16 * 41];
+    __shared__ float2 loss_w[kFbWaves];
     if (!gs->active) return;
     for (int i = threadIdx.x; i < kGFwdSize / 8; i += blockDim.x)
         reinterpret_cast<u32x4_t*>(wf_lds)[i] = reinterpret_cast<const u32x4_t*>(wf)[i];
@@ -259,10 +263,10 @@ __global__ __launch_bounds__(256) void k_guide_fb(const uint16_t* __restrict__ w
     float* dlw = dl[wv];
     const uint32_t ld = tb.ld;
     float loss_acc = 0.0f, w_acc = 0.0f;
-    const uint32_t waves = gridDim.x * 4;
-    for (uint32_t tile = blockIdx.x * 4 + wv; tile * 16 < tb.ncols; tile += waves) {
+    const uint32_t nw = blockDim.x / 64, waves = gridDim.x * nw;
+    for (uint32_t tile = blockIdx.x * nw + wv; tile * 16 < tb.ncols; tile += waves) {
         const uint32_t q = tile * 16 + r;
-        const float4 x0 = tb.tb[0][q], x1 = tb.tb[1][q];
+        const float4 x0 = tb.tb[0][q], x1 = tb.tb[1][q], dir = tb.tb[2][q];
         const float xin[7] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z};
         FbHook hook;
 #pragma unroll
@@ -278,45 +282,57 @@ __global__ __launch_bounds__(256) void k_guide_fb(const uint16_t* __restrict__ w
                 if (u < kGOut) dlw[r * 41 + u] = out[mt][0][k];
             }
         wave_lds_sync();
-        if (g == 0) {
-            float o[kGOut];
-#pragma unroll
-            for (int u = 0; u < kGOut; u++) o[u] = dlw[r * 41 + u];
-            GuideMix m;
-            mix_from_outputs([&](int u) { return o[u]; }, m);
-            const float4 dir = tb.tb[2][q];
+        {
+            // responsibilities and -w * d log q / d outputs; this lane's lobes are 2g and 2g + 1
+            const float* orow = dlw + r * 41;
+            const auto o = [orow](int u) { return orow[u]; };
+            const float ls = mix_log_norm(o);
             const float w = q < b_eff ? x1.w : 0.0f;
-            // responsibilities and -w * d log q / d outputs
-            float t[kGLobes], cs[kGLobes], mxv = -3.0e38f;
+            GuideLobe lb[2];
+            float logpi[2], cs[2], tk2[2], mraw[2][3], rr[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int k = 2 * g + j;
+                lb[j] = mix_lobe(o, k, ls);
+                logpi[j] = o(5 * k) - ls;
+                const float lognorm = lb[j].logw - logpi[j];
+                cs[j] = lb[j].mx * dir.x + lb[j].my * dir.y + lb[j].mz * dir.z;
+                tk2[j] = logpi[j] + lognorm + lb[j].kappa * (cs[j] - 1.0f);
+#pragma unroll
+                for (int a = 0; a < 3; a++) mraw[j][a] = o(5 * k + 1 + a);
+                rr[j] = o(5 * k + 4);
+            }
+            float t[kGLobes], mxv = -3.0e38f;
 #pragma unroll
             for (int k = 0; k < kGLobes; k++) {
-                cs[k] = m.mx[k] * dir.x + m.my[k] * dir.y + m.mz[k] * dir.z;
-                t[k] = m.logpi[k] + m.lognorm[k] + m.kappa[k] * (cs[k] - 1.0f);
+                t[k] = __shfl(tk2[k & 1], (k >> 1) * 16 + r);
                 mxv = fmaxf(mxv, t[k]);
             }
             float s = 0.0f;
 #pragma unroll
             for (int k = 0; k < kGLobes; k++) s += __expf(t[k] - mxv);
             const float lq = mxv + __logf(s);
-            if (w > 0.0f) {
+            if (g == 0 && w > 0.0f) {
                 loss_acc += -w * lq;
                 w_acc += w;
             }
+            wave_lds_sync();  // every lane has read the outputs its sample's other lanes overwrite
 #pragma unroll
-            for (int k = 0; k < kGLobes; k++) {
-                const float gam = __expf(t[k] - lq), pi = __expf(m.logpi[k]), kap = m.kappa[k];
-                dlw[r * 41 + 5 * k] = -w * (gam - pi);
-                const float mlen = sqrtf(fmaxf(o[5 * k + 1] * o[5 * k + 1] + o[5 * k + 2] * o[5 * k + 2] +
-                                                   o[5 * k + 3] * o[5 * k + 3], 1.0e-12f));
+            for (int j = 0; j < 2; j++) {
+                const int k = 2 * g + j;
+                const float gam = __expf(tk2[j] - lq), pi = __expf(logpi[j]), kap = lb[j].kappa;
+                float* out_k = dlw + r * 41 + 5 * k;
+                out_k[0] = -w * (gam - pi);
+                const float mlen = sqrtf(fmaxf(mraw[j][0] * mraw[j][0] + mraw[j][1] * mraw[j][1] +
+                                                   mraw[j][2] * mraw[j][2], 1.0e-12f));
                 const float sc = -w * gam * kap / mlen;
-                dlw[r * 41 + 5 * k + 1] = sc * (dir.x - cs[k] * m.mx[k]);
-                dlw[r * 41 + 5 * k + 2] = sc * (dir.y - cs[k] * m.my[k]);
-                dlw[r * 41 + 5 * k + 3] = sc * (dir.z - cs[k] * m.mz[k]);
-                const float rr = o[5 * k + 4];
-                const bool inside = rr > kGLogKappaLo && rr < kGLogKappaHi;
+                out_k[1] = sc * (dir.x - cs[j] * lb[j].mx);
+                out_k[2] = sc * (dir.y - cs[j] * lb[j].my);
+                out_k[3] = sc * (dir.z - cs[j] * lb[j].mz);
+                const bool inside = rr[j] > kGLogKappaLo && rr[j] < kGLogKappaHi;
                 const float tk = 2.0f * kap;
-                const float dr = 1.0f - tk / expm1f(tk) + kap * (cs[k] - 1.0f);
-                dlw[r * 41 + 5 * k + 4] = inside ? -w * gam * dr : 0.0f;
+                const float dr = 1.0f - tk / expm1f(tk) + kap * (cs[j] - 1.0f);
+                out_k[4] = inside ? -w * gam * dr : 0.0f;
             }
         }
         wave_lds_sync();
@@ -350,7 +366,7 @@ __global__ __launch_bounds__(256) void k_guide_fb(const uint16_t* __restrict__ w
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int mt = 0; mt < 4; mt++) {
-                    const u32x4_t a = ld16(wbt + wt_off[l - 2] + (16 * mt + r) * 64 + 32 * c + 8 * g);
+                    const u32x4_t a = ld16(wbt + wt_off[l - 2] + (16 * mt + r) * kGRowH + 32 * c + 8 * g);
                     acc[mt] = mfma_bf16(a, bd[c], acc[mt]);
                 }
             u32x4_t nd[2];
@@ -360,36 +376,60 @@ __global__ __launch_bounds__(256) void k_guide_fb(const uint16_t* __restrict__ w
             bd[1] = nd[1];
         }
     }
-    // one atomic per wave for the loss monitor
+    // the loss monitor: one partial per block, summed by k_guide_adam in a fixed order.  (An atomic per
+    // wave on the two sums is a compare-and-swap loop on one address: 42 us of every step with 1,024
+    // waves, 108 us with 4,096.)
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         loss_acc += __shfl_xor(loss_acc, o);
         w_acc += __shfl_xor(w_acc, o);
     }
-    if (lane == 0) {
-        atomicAdd(&gs->loss_sum, loss_acc);
-        atomicAdd(&gs->weight_sum, w_acc);
+    if (lane == 0) loss_w[wv] = make_float2(loss_acc, w_acc);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float2 t = loss_w[0];
+        for (uint32_t v = 1; v < nw; v++) t = make_float2(t.x + loss_w[v].x, t.y + loss_w[v].y);
+        loss_part[blockIdx.x] = t;
     }
 }
 
-// Weight gradients.  blockIdx.x = tile: 0..3 layer 1 (64 code columns each), 4..6 layers
-// 2..4, 7 layer 5; blockIdx.y = sample range.  One wave accumulates up to 64 x 64 outputs
-// over its range, 32 samples at a time: the query-major rows are staged into LDS
-// transposed (unit-major), so each MFMA operand is one 16-byte LDS read of 8 samples.
-constexpr int kDwStride = 40;  // LDS row stride in bf16 (32 samples + pad, keeps 16 B alignment)
+// Weight gradients.  A block takes one tile (0..3 layer 1, 64 code columns each; 4..6 layers 2..4; 7
+// layer 5) of one sample range.  A block of four waves accumulates up to 64 x 64 outputs
+// over its range, 128 samples at a time: each wave stages 32 of them into LDS transposed (unit-major,
+// so each MFMA operand is one 16-byte LDS read of 8 samples), then every wave takes the four chunks
+// in order for its 16 columns, so an output's products are added in sample order as one wave would.
+// Bound below 2^16 samples: the staging's serial latency.  One wave a block, writing 2 bytes at a time (64 conflicted LDS
+// writes an operand), took 158 us for 2^18 samples and 73 us for a batch of 4,096; 8-byte writes of four
+// samples, the rows of the next chunks in flight and four waves a block take 105 and 27 us.  At 2^18 it
+// is bound by its reads: 303 MB (410 MB before the block order below), 3.2 TB/s.
+// LDS offset, in bf16, of unit u's samples s .. s + 3 (s a multiple of 4) of a chunk of 32: rows of 64 bytes
+// in pairs, the pair's eight 16-byte pieces permuted by the row, so that the 16 rows of a read and the 8
+// chunks of a write each meet all banks evenly and four blocks fit a CU (padded rows held three).
+__host__ __device__ constexpr int dw_at(int u, int s) {
+    return (u >> 1) * 64 + (((((u & 1) << 2) | (s >> 3)) ^ ((u >> 1) & 3) ^ ((u >> 3) & 7)) * 8) + (s & 7);
+}
+constexpr int kDwTile = 64 * 32;
+constexpr int kDwWaves = 4;
 
-__global__ __launch_bounds__(64) void k_guide_dw(TrainBufs tb, const GuideState* __restrict__ gs, float* partial,
-                                                 uint32_t cols_per_split) {
-    __shared__ __attribute__((aligned(16))) uint16_t sa[64 * kDwStride];
-    __shared__ __attribute__((aligned(16))) uint16_t sb[64 * kDwStride];
+__global__ __launch_bounds__(64 * kDwWaves) void k_guide_dw(TrainBufs tb, const GuideState* __restrict__ gs, float* partial,
+                                                           uint32_t cols_per_split, uint32_t splits) {
+    __shared__ __attribute__((aligned(16))) uint16_t sa[kDwWaves][kDwTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sb[kDwWaves][kDwTile];
     if (!gs->active) return;
-    const int tile = blockIdx.x, lane = __lane_id(), g = lane >> 4, r = lane & 15;
+    // Blocks go to the 8 XCDs in turn: a range's 8 tiles take every eighth block, so that layer 1's four
+    // find its deltas in one L2.  The last ranges come first: they were written last and are what the
+    // 256 MB Infinity Cache still holds of a large batch's 302 MB.
+    const uint32_t lin = blockIdx.x, whole = splits & ~7u, grp = lin / 64u;
+    const uint32_t tile = lin < 8u * whole ? (lin / 8u) & 7u : (lin - 8u * whole) & 7u;
+    const uint32_t from_end = lin < 8u * whole ? grp * 8u + (lin & 7u) : whole + (lin - 8u * whole) / 8u;
+    const uint32_t split = splits - 1u - from_end;
+    const int lane = __lane_id(), wv = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
     int layer, kbase = 0;
     if (tile < 4) {
         layer = 1;
-        kbase = 64 * tile;
+        kbase = 64 * (int)tile;
     } else {
-        layer = tile - 2;
+        layer = (int)tile - 2;
     }
     const int K = layer == 1 ? kGEnc : kGHid;       // columns of W (row length of the B rows)
     const int nvalid = layer == 5 ? kGOut : kGHid;
@@ -399,75 +439,88 @@ __global__ __launch_bounds__(64) void k_guide_dw(TrainBufs tb, const GuideState*
     const size_t ld = tb.ld;
     const uint16_t* A = tb.dz + (size_t)(layer - 1) * ld * 64;                       // [q][64]
     const uint16_t* B = tb.act + (size_t)(layer == 1 ? 0 : layer - 2) * ld * 64;  // [q][64] (layers 2..5)
-    const uint32_t q_lo = blockIdx.y * cols_per_split, q_hi = min(tb.ncols, q_lo + cols_per_split);
-    f32x4_t acc[4][4];
+    const uint32_t q_lo = split * cols_per_split, q_hi = min(tb.ncols, q_lo + cols_per_split);
+    const int kt = wv;  // this wave's 16 columns
+    f32x4_t acc[4];
     float bsum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+    for (int mt = 0; mt < 4; mt++) acc[mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    // This lane stages 4 samples of one 8-slot chunk: slot by slot the four 16-bit values of the
+    // samples make one 8-byte write.
+    const int ch = lane & 7, s4 = 4 * (lane >> 3);
+    const bool b_used = 8 * ch < ncols;
+    const int col = kbase + 8 * ch, xc = col >> 5, xg = (col >> 3) & 3;
+    u32x4_t va[4], vb[4];
+    float xv[4];
+    auto fetch = [&](uint32_t q0) {
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++) acc[mt][kt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t q0 = q_lo; q0 < q_hi; q0 += 32) {
-        // stage: 32 samples x 64 slots of A and 32 x ncols of B, written transposed
+        for (int i = 0; i < 4; i++) {
+            const size_t q = q0 + s4 + i;
+            va[i] = *reinterpret_cast<const u32x4_t*>(A + q * 64 + 8 * ch);
+            if (layer == 1) xv[i] = reinterpret_cast<const float*>(tb.tb[xc >> 2] + q)[xc & 3];
+            else vb[i] = *reinterpret_cast<const u32x4_t*>(B + q * 64 + 8 * ch);
+        }
+    };
+    auto transpose_to = [&](uint16_t* dst, const u32x4_t (&v)[4]) {
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int e = it * 64 + lane;        // 256 vectors of 8 bf16: sample e / 8, chunk e % 8
-            const int qs = e >> 3, ch = e & 7;
-            const u32x4_t va = *reinterpret_cast<const u32x4_t*>(A + (size_t)(q0 + qs) * 64 + 8 * ch);
-            u32x4_t vb = u32x4_t{0u, 0u, 0u, 0u};
-            if (8 * ch < ncols) {
-                if (layer == 1) {
-                    // code bins col .. col + 7 of the sample: input col / 32, bins col % 32 ..,
-                    // computed as the forward pass of k_guide_fb computed them
-                    const int col = kbase + 8 * ch, c = col >> 5;
-                    const float* xr = reinterpret_cast<const float*>(tb.tb[c >> 2] + (q0 + qs));
-                    vb = blob8(xr[c & 3], (col >> 3) & 3);
-                } else {
-                    vb = *reinterpret_cast<const u32x4_t*>(B + (size_t)(q0 + qs) * K + 8 * ch);
-                }
+        for (int j = 0; j < 8; j++) {
+            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low halves of two words
+            uint2 p;
+            p.x = __builtin_amdgcn_perm(v[1][j >> 1], v[0][j >> 1], sel);
+            p.y = __builtin_amdgcn_perm(v[3][j >> 1], v[2][j >> 1], sel);
+            *reinterpret_cast<uint2*>(dst + dw_at(8 * ch + j, s4)) = p;
+        }
+    };
+    const uint32_t own = 32u * (uint32_t)wv;  // this wave's chunk of the 128 samples
+    if (q_lo + own < q_hi) fetch(q_lo + own);
+    for (uint32_t q0 = q_lo; q0 < q_hi; q0 += 32u * kDwWaves) {
+        if (q0 + own < q_hi) {
+            if (layer == 1) {
+                // code bins col .. col + 7 of the sample: input col / 32, bins col % 32 ..,
+                // computed as the forward pass of k_guide_fb computed them
+#pragma unroll
+                for (int i = 0; i < 4; i++) vb[i] = b_used ? blob8(xv[i], xg) : u32x4_t{0u, 0u, 0u, 0u};
             }
+            transpose_to(sa[wv], va);
+            transpose_to(sb[wv], vb);
+        }
+        if (q0 + own + 32u * kDwWaves < q_hi) fetch(q0 + own + 32u * kDwWaves);  // in flight during the products
+        __syncthreads();
+        const int nc = (int)min((uint32_t)kDwWaves, (q_hi - q0) / 32u);
+        for (int c = 0; c < nc; c++) {
+            u32x4_t a[4];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const uint32_t wa = va[j >> 1], wbv = vb[j >> 1];
-                sa[(8 * ch + j) * kDwStride + qs] = (uint16_t)((j & 1) ? (wa >> 16) : (wa & 0xffffu));
-                sb[(8 * ch + j) * kDwStride + qs] = (uint16_t)((j & 1) ? (wbv >> 16) : (wbv & 0xffffu));
+            for (int mt = 0; mt < 4; mt++) a[mt] = *reinterpret_cast<const u32x4_t*>(sa[c] + dw_at(16 * mt + r, 8 * g));
+            const u32x4_t b = *reinterpret_cast<const u32x4_t*>(sb[c] + dw_at(16 * kt + r, 8 * g));
+            if (kt < nkt) {
+#pragma unroll
+                for (int mt = 0; mt < 4; mt++)
+                    if (mt < nmt) acc[mt] = mfma_bf16(a[mt], b, acc[mt]);
+            }
+            if (kbase == 0 && wv == 0) {
+#pragma unroll
+                for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) bsum[mt] += bf16_lo(a[mt][j]) + bf16_hi(a[mt][j]);
             }
         }
-        wave_lds_sync();
-        u32x4_t a[4], b[4];
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++) a[mt] = *reinterpret_cast<const u32x4_t*>(sa + (16 * mt + r) * kDwStride + 8 * g);
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++) b[kt] = *reinterpret_cast<const u32x4_t*>(sb + (16 * kt + r) * kDwStride + 8 * g);
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int kt = 0; kt < 4; kt++)
-                if (mt < nmt && kt < nkt) acc[mt][kt] = mfma_bf16(a[mt], b[kt], acc[mt][kt]);
-        if (kbase == 0) {
-#pragma unroll
-            for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) bsum[mt] += bf16_lo(a[mt][j]) + bf16_hi(a[mt][j]);
-        }
-        wave_lds_sync();
+        __syncthreads();
     }
     // Rows of A are slots of the layer's outputs (natural order for layer 5); columns of B
     // are code bins (layer 1) or slots of the previous layer's outputs.
     const int offW[5] = {kGOffW1, kGOffW2, kGOffW3, kGOffW4, kGOffW5};
     const int offB[5] = {kGOffB1, kGOffB2, kGOffB3, kGOffB4, kGOffB5};
-    float* out = partial + (size_t)blockIdx.y * kGParams;
+    float* out = partial + (size_t)split * kGParams;
 #pragma unroll
     for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int sn = 16 * mt + 4 * g + i, sk = 16 * kt + r;
-                const int n = layer == 5 ? sn : slot_unit(sn);
-                const int k = layer == 1 ? kbase + sk : slot_unit(sk);
-                if (mt < nmt && kt < nkt && n < nvalid) out[offW[layer - 1] + n * K + k] = acc[mt][kt][i];
-            }
-    if (kbase == 0) {
+        for (int i = 0; i < 4; i++) {
+            const int sn = 16 * mt + 4 * g + i, sk = 16 * kt + r;
+            const int n = layer == 5 ? sn : slot_unit(sn);
+            const int k = layer == 1 ? kbase + sk : slot_unit(sk);
+            if (mt < nmt && kt < nkt && n < nvalid) out[offW[layer - 1] + n * K + k] = acc[mt][i];
+        }
+    if (kbase == 0 && wv == 0) {
 #pragma unroll
         for (int mt = 0; mt < 4; mt++) {
             float s = bsum[mt];
@@ -536,11 +589,27 @@ __global__ void k_guide_gnorm(const float* __restrict__ gnorm_part, GuideState* 
     gs->gnorm2 = t;
 }
 
-__global__ void k_guide_adam(float* params, float* m, float* v, const float* __restrict__ partial, int splits,
-                             const GuideState* __restrict__ gs, AdamCfg cfg, float* grad_out, uint16_t* wf, uint16_t* wb,
-                             float* bias) {
+static_assert(kGParams % 256 != 0 && kGParams % 256 <= 192, "the last block of k_guide_adam has a spare wave");
+__global__ __launch_bounds__(256) void k_guide_adam(float* params, float* m, float* v, const float* __restrict__ partial, int splits,
+                             GuideState* gs, AdamCfg cfg, float* grad_out, uint16_t* wf, uint16_t* wb, float* bias,
+                             const float2* __restrict__ loss_part, int n_loss) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kGParams || !gs->active) return;
+    if (!gs->active) return;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x >= 192) {
+        // the last block's last wave holds no parameters: k_guide_fb's loss partials
+        float2 t = make_float2(0.0f, 0.0f);
+        for (int i = (int)threadIdx.x - 192; i < n_loss; i += 64) t = make_float2(t.x + loss_part[i].x, t.y + loss_part[i].y);
+        for (int o = 32; o > 0; o >>= 1) {
+            t.x += __shfl_xor(t.x, o);
+            t.y += __shfl_xor(t.y, o);
+        }
+        if (threadIdx.x == 192) {
+            gs->loss_sum = t.x;
+            gs->weight_sum = t.y;
+        }
+        return;
+    }
+    if (p >= kGParams) return;
     float s = 0.0f;
     for (int k = 0; k < splits; k++) s += partial[(size_t)k * kGParams + p];
     float gr = s / (float)gs->b_eff;
@@ -646,12 +715,17 @@ int launch_guide_step(const GuideBufsDev& gb, const TrainBufs& tb, const GuideNe
     hipLaunchKernelGGL(k_guide_step_begin, dim3(1), dim3(64), 0, st, gb.gs, tb.batch, net ? net->rec_cap : 0u, seed,
                        direct_n, bump_t ? 1u : 0u);
     if (!direct_n) hipLaunchKernelGGL(k_guide_batch, dim3(1024), dim3(256), 0, st, *net, (const GuideState*)gb.gs, tb);
-    const uint32_t fb_blocks = std::max(1u, std::min((uint32_t)gb.grid, (tb.ncols / 16 + 3) / 4));
-    hipLaunchKernelGGL(k_guide_fb, dim3(fb_blocks), dim3(256), 0, st, (const uint16_t*)gb.wf, (const float*)gb.bias,
-                       (const uint16_t*)gb.wb, tb, gb.gs);
+    // Four tiles a block at least, and one wave a tile up to 16: a small batch spreads over the CUs first
+    // (us by waves a block, 8 / 16: 2^14 samples 19 / 23, 2^16 24 / 21, 2^18 91 / 87).
+    const uint32_t tiles = tb.ncols / 16;
+    const uint32_t fb_blocks = std::max(1u, std::min((uint32_t)gb.grid, (tiles + 3) / 4));
+    const uint32_t fb_waves = std::min((uint32_t)kFbWaves, std::max(4u, (tiles + fb_blocks - 1) / fb_blocks));
+    hipLaunchKernelGGL(k_guide_fb, dim3(fb_blocks), dim3(64 * fb_waves), 0, st, (const uint16_t*)gb.wf, (const float*)gb.bias,
+                       (const uint16_t*)gb.wb, tb, (const GuideState*)gb.gs, gb.loss_part);
     const uint32_t cps = kGuideColsPerSplit;
     const uint32_t splits = (tb.ncols + cps - 1) / cps;
-    hipLaunchKernelGGL(k_guide_dw, dim3(8, splits), dim3(64), 0, st, tb, (const GuideState*)gb.gs, gb.partial, cps);
+    hipLaunchKernelGGL(k_guide_dw, dim3(8 * splits), dim3(64 * kDwWaves), 0, st, tb, (const GuideState*)gb.gs, gb.partial, cps,
+                       splits);
     const bool clip = kGuideClip > 0.0f && !grad_out;
     const float* red = gb.partial;  // the rows Adam sums
     int nred = (int)splits;
@@ -667,7 +741,7 @@ int launch_guide_step(const GuideBufsDev& gb, const TrainBufs& tb, const GuideNe
         nred = kPsumGroups;
     }
     hipLaunchKernelGGL(k_guide_adam, dim3((kGParams + 255) / 256), dim3(256), 0, st, gb.params, gb.m, gb.v, red, nred,
-                       (const GuideState*)gb.gs, cfg, grad_out, gb.wf, gb.wb, gb.bias);
+                       gb.gs, cfg, grad_out, gb.wf, gb.wb, gb.bias, (const float2*)gb.loss_part, (int)fb_blocks);
     SPK_CHECK_HIP(hipGetLastError());
     return SPK_OK;
 }

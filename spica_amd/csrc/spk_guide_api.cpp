@@ -26,6 +26,7 @@ spk::GuideBufsDev spk_guide::bufs() const {
     b.partial = partial.as<float>();
     b.psum = psum.as<float>();
     b.gnorm_part = gnorm_part.as<float>();
+    b.loss_part = loss_part.as<float2>();
     b.gs = state.as<GuideState>();
     b.grid = cus;
     return b;
@@ -203,7 +204,8 @@ int spk_guide_create(int device, const spk_guide_opts* opts, spk_guide** out) {
         (rc = g->wf.alloc(kGFwdSize * 2)) || (rc = g->wb.alloc(kGBwdSize * 2)) || (rc = g->bias.alloc(kGBiasSize * 4)) ||
         (rc = g->partial.alloc(splits * kGParams * 4)) || (rc = g->psum.alloc((size_t)kPsumGroups * kGParams * 4)) ||
         (rc = g->state.alloc(sizeof(GuideState))) ||
-        (rc = g->grad.alloc(kGParams * 4)) || (rc = g->gnorm_part.alloc(kGnormBlocks * 4)))
+        (rc = g->grad.alloc(kGParams * 4)) || (rc = g->gnorm_part.alloc(kGnormBlocks * 4)) ||
+        (rc = g->loss_part.alloc((size_t)std::max(1, g->cus) * 8)))
         return rc;
     for (int k = 0; k < 3; k++)
         if ((rc = g->tb[k].alloc(B * 16))) return rc;
@@ -229,7 +231,7 @@ int spk_guide_destroy(spk_guide* g) {
         (void)hipStreamDestroy(g->stream);
     }
     DevBuf* b[] = {&g->params, &g->m, &g->v, &g->wf, &g->wb, &g->bias, &g->partial, &g->psum, &g->state, &g->grad,
-                   &g->gnorm_part, &g->tb[0], &g->tb[1], &g->tb[2], &g->act, &g->dz};
+                   &g->gnorm_part, &g->loss_part, &g->tb[0], &g->tb[1], &g->tb[2], &g->act, &g->dz};
     for (DevBuf* x : b) x->release();
     delete g;
     return SPK_OK;

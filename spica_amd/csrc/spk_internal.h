@@ -232,6 +232,7 @@ struct GuideBufsDev {
     float* bias;
     float* partial;     // [splits][kGParams]
     float* psum;        // [kPsumGroups][kGParams]: partial folded in fixed groups of ranges
+    float2* loss_part;  // [grid] k_guide_fb's loss and weight sums per block
     float* gnorm_part;  // [kGnormBlocks] squared-norm partials of one step's gradient
     GuideState* gs;
     int grid;           // persistent blocks for the training kernel (compute units)
@@ -260,7 +261,7 @@ struct spk_guide {
     int device = 0;
     hipStream_t stream = nullptr;       // for the stand-alone entry points
     spk_guide_opts opts;
-    spk::DevBuf params, m, v, wf, wb, bias, partial, psum, state, grad, gnorm_part;
+    spk::DevBuf params, m, v, wf, wb, bias, partial, psum, state, grad, gnorm_part, loss_part;
     spk::DevBuf tb[3], act, dz;
     uint32_t bcap = 0;                  // batch capacity (samples)
     int cus = 256;                      // compute units of the device
