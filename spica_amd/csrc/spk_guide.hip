@@ -71,11 +71,13 @@ __global__ void k_guide_images(const float* __restrict__ params, uint16_t* wf, u
 
 // ---- evaluation (C-ABI checks) ----------------------------------------------------------------------
 // Block of 256 = 4 waves, each taking 64 queries per iteration with the weights in LDS,
-// exactly as the render kernel does.
+// exactly as the render kernel does.  Inputs and results are the caller's own layouts (x [n][7],
+// aux [n][3], out_dir [n][3]), so nothing is packed on the host.
 template <int MODE>  // 0: outputs + log pdf of given directions; 1: sample directions
 __global__ __launch_bounds__(256) void k_guide_eval(const uint16_t* __restrict__ wf, const float* __restrict__ bias,
-                                                    int64_t n, const float4* __restrict__ x, const float4* __restrict__ aux,
-                                                    float* __restrict__ out_raw, float4* __restrict__ res) {
+                                                    int64_t n, const float* __restrict__ x, const float* __restrict__ aux,
+                                                    float* __restrict__ out_raw, float* __restrict__ out_dir,
+                                                    float* __restrict__ out_pdf) {
     __shared__ __attribute__((aligned(16))) uint16_t w_lds[kGFwdSize];
     __shared__ float b_lds[kGBiasSize];
     __shared__ float obuf[4][64 * 41];
@@ -89,18 +91,8 @@ __global__ __launch_bounds__(256) void k_guide_eval(const uint16_t* __restrict__
     for (int64_t base = ((int64_t)blockIdx.x * 4 + wv) * 64; base < n; base += waves * 64) {
         const int64_t i = base + lane;
         const bool active = i < n;
-        float4 x0 = make_float4(0.5f, 0.5f, 0.5f, 0.5f), x1 = make_float4(0.5f, 0.5f, 0.5f, 0.0f);
-        if (active) {
-            x0 = x[2 * i];
-            x1 = x[2 * i + 1];
-        }
-        ob[lane * 8 + 0] = x0.x;
-        ob[lane * 8 + 1] = x0.y;
-        ob[lane * 8 + 2] = x0.z;
-        ob[lane * 8 + 3] = x0.w;
-        ob[lane * 8 + 4] = x1.x;
-        ob[lane * 8 + 5] = x1.y;
-        ob[lane * 8 + 6] = x1.z;
+#pragma unroll
+        for (int d = 0; d < kGIn; d++) ob[lane * 8 + d] = active ? x[kGIn * i + d] : 0.5f;
         wave_lds_sync();
         f32x4_t out[3][4];
         NoHook hook;
@@ -122,12 +114,15 @@ __global__ __launch_bounds__(256) void k_guide_eval(const uint16_t* __restrict__
                 for (int u = 0; u < kGOut; u++) out_raw[i * kGOut + u] = o[u];
             GuideMix mix;
             mix_from_outputs([&](int u) { return o[u]; }, mix);
-            const float4 a = aux[i];
+            const float3 a = make_float3(aux[3 * i], aux[3 * i + 1], aux[3 * i + 2]);
             if (MODE == 0) {
-                res[i] = make_float4(mix_log_pdf(mix, a.x, a.y, a.z), 0.0f, 0.0f, 0.0f);
+                if (out_pdf) out_pdf[i] = mix_log_pdf(mix, a.x, a.y, a.z);
             } else {
-                float3 d = mix_sample(mix, a.x, a.y, a.z);
-                res[i] = make_float4(d.x, d.y, d.z, __expf(mix_log_pdf(mix, d.x, d.y, d.z)));
+                const float3 d = mix_sample(mix, a.x, a.y, a.z);
+                out_dir[3 * i] = d.x;
+                out_dir[3 * i + 1] = d.y;
+                out_dir[3 * i + 2] = d.z;
+                if (out_pdf) out_pdf[i] = __expf(mix_log_pdf(mix, d.x, d.y, d.z));
             }
         }
         wave_lds_sync();
@@ -160,6 +155,24 @@ __global__ void k_guide_step_begin(GuideState* gs, uint32_t batch, uint32_t rec_
         gs->gnorm_ema = ema > 0.0f ? 0.9f * ema + 0.1f * fminf(norm, kGuideClip * ema) : norm;
         gs->gnorm2 = 0.0f;
     }
+}
+
+// A caller's batch (x [n][7], dirs [n][3], weight [n]) as training columns; columns beyond n carry weight 0.
+__global__ void k_guide_pack(const float* __restrict__ x, const float* __restrict__ dirs, const float* __restrict__ weight,
+                             uint32_t n, TrainBufs tb) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= tb.ncols) return;
+    float4 t0 = make_float4(0.5f, 0.5f, 0.5f, 0.5f), t1 = make_float4(0.5f, 0.5f, 0.5f, 0.0f),
+           t2 = make_float4(0.0f, 0.0f, 1.0f, 0.0f);
+    if (i < n) {
+        const float* xi = x + kGIn * (size_t)i;
+        t0 = make_float4(xi[0], xi[1], xi[2], xi[3]);
+        t1 = make_float4(xi[4], xi[5], xi[6], weight[i]);
+        t2 = make_float4(dirs[3 * (size_t)i], dirs[3 * (size_t)i + 1], dirs[3 * (size_t)i + 2], 0.0f);
+    }
+    tb.tb[0][i] = t0;
+    tb.tb[1][i] = t1;
+    tb.tb[2][i] = t2;
 }
 
 __device__ __forceinline__ float safe_ratio(float a, float b) { return b > 0.0f ? a / b : 0.0f; }
@@ -640,12 +653,21 @@ int launch_guide_images(const float* params, uint16_t* wf, uint16_t* wb, float* 
     return SPK_OK;
 }
 
-int launch_guide_eval(int mode, const uint16_t* wf, const float* bias, int64_t n, const float4* x, const float4* aux,
-                      float* out_raw, float4* res, int grid, hipStream_t st) {
+int launch_guide_eval(int mode, const uint16_t* wf, const float* bias, int64_t n, const float* x, const float* aux,
+                      float* out_raw, float* out_dir, float* out_pdf, int grid, hipStream_t st) {
+    // no more blocks than have queries: each copies the 64 KB of weights
+    const int g = (int)std::min<int64_t>(grid, (n + 255) / 256);
     if (mode == 0)
-        hipLaunchKernelGGL(k_guide_eval<0>, dim3(grid), dim3(256), 0, st, wf, bias, n, x, aux, out_raw, res);
+        hipLaunchKernelGGL(k_guide_eval<0>, dim3(g), dim3(256), 0, st, wf, bias, n, x, aux, out_raw, out_dir, out_pdf);
     else
-        hipLaunchKernelGGL(k_guide_eval<1>, dim3(grid), dim3(256), 0, st, wf, bias, n, x, aux, out_raw, res);
+        hipLaunchKernelGGL(k_guide_eval<1>, dim3(g), dim3(256), 0, st, wf, bias, n, x, aux, out_raw, out_dir, out_pdf);
+    SPK_CHECK_HIP(hipGetLastError());
+    return SPK_OK;
+}
+
+int launch_guide_pack(const float* x, const float* dirs, const float* weight, uint32_t n, const TrainBufs& tb,
+                      hipStream_t st) {
+    hipLaunchKernelGGL(k_guide_pack, dim3((tb.ncols + 255) / 256), dim3(256), 0, st, x, dirs, weight, n, tb);
     SPK_CHECK_HIP(hipGetLastError());
     return SPK_OK;
 }

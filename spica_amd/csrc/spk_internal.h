@@ -242,8 +242,10 @@ constexpr int kPsumGroups = 16;
 constexpr int kGnormBlocks = (kGParams + 255) / 256;
 
 int launch_guide_images(const float* params, uint16_t* wf, uint16_t* wb, float* bias, hipStream_t st);
-int launch_guide_eval(int mode, const uint16_t* wf, const float* bias, int64_t n, const float4* x, const float4* aux,
-                      float* out_raw, float4* res, int grid, hipStream_t st);
+int launch_guide_eval(int mode, const uint16_t* wf, const float* bias, int64_t n, const float* x, const float* aux,
+                      float* out_raw, float* out_dir, float* out_pdf, int grid, hipStream_t st);
+int launch_guide_pack(const float* x, const float* dirs, const float* weight, uint32_t n, const TrainBufs& tb,
+                      hipStream_t st);
 // Training records of one round in a fixed order: sorted by (sample, pixel, depth) into out[0..4], so
 // the batches, and with them the trained network, do not depend on the order in which the
 // queue appends stored the records.  keys/idx hold 2 * cap entries each (input and sorted).
@@ -263,6 +265,7 @@ struct spk_guide {
     spk_guide_opts opts;
     spk::DevBuf params, m, v, wf, wb, bias, partial, psum, state, grad, gnorm_part, loss_part;
     spk::DevBuf tb[3], act, dz;
+    spk::DevBuf stage;                  // callers' arrays on the device, kept between calls
     uint32_t bcap = 0;                  // batch capacity (samples)
     int cus = 256;                      // compute units of the device
     int64_t steps = 0;                  // Adam steps launched
