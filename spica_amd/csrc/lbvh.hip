@@ -7,17 +7,14 @@
 //   2. one thread per internal node finds the node's key range and split from the
 //      common-prefix lengths of neighbouring codes (ties broken by index), giving a
 //      binary radix tree whose node i covers a contiguous range of sorted triangles;
-//   3. boxes bottom-up: each leaf walks to the root, the second thread to reach a node
-//      (an atomic counter per node) merges its children's boxes and computes the node's
-//      SAH cost; a subtree of at most max_leaf triangles whose cost as one leaf is no
-//      higher than as a subtree is marked to collapse (the rule of Karras and Aila, "Fast
-//      parallel construction of high-quality BVHs", HPG 2013);
-//   4. treelet restructuring (Karras and Aila 2013): bottom-up sweeps in which every node
-//      of at least kTreeletMinTris triangles takes the treelet of its up to 7 largest
-//      descendants and rebuilds the treelet's inner topology with the cheapest SAH cost
-//      (spk_treelet.h), followed by a top-down pass, one level per launch, that gives every
-//      subtree its contiguous range of the final triangle order (depth first);
-//   5. boxes, SAH costs and the leaf collapse of step 3 again over the restructured tree;
+//   3. treelet restructuring (Karras and Aila, "Fast parallel construction of high-quality BVHs", HPG
+//      2013): bottom-up sweeps in which every node of at least kTreeletMinTris triangles takes the
+//      treelet of its up to 7 largest descendants and rebuilds the treelet's inner topology with the
+//      cheapest SAH cost (spk_treelet.h);
+//   4. a top-down pass that gives every subtree its contiguous range of the final triangle order
+//      (depth first);
+//   5. boxes and SAH costs bottom-up; a subtree of at most max_leaf triangles whose cost as one leaf is
+//      no higher than as a subtree is marked to collapse (the rule of Karras and Aila);
 //   6. emit binary nodes (collapsed subtrees as leaves over their contiguous ranges), then
 //      renumber the reachable nodes depth first on the host; the scene then collapses
 //      them into 4-wide nodes like the SAH tree's.
@@ -73,7 +70,7 @@ __device__ __forceinline__ int delta(const uint64_t* __restrict__ c, int n, int 
 }
 
 // Internal nodes 0 .. n-2; child ids < n-1 are internal nodes, id (n-1) + k is leaf k.
-__global__ void k_hierarchy(const uint64_t* __restrict__ c, int n, int2* child, int2* range, int* parent) {
+__global__ void k_hierarchy(const uint64_t* __restrict__ c, int n, int2* child, int2* range, int* parent, int* size) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n - 1; i += gridDim.x * blockDim.x) {
         const int d = (delta(c, n, i, i + 1) - delta(c, n, i, i - 1)) >= 0 ? 1 : -1;
         const int dmin = delta(c, n, i, i - d);
@@ -95,6 +92,7 @@ __global__ void k_hierarchy(const uint64_t* __restrict__ c, int n, int2* child, 
         const int right = hi == gamma + 1 ? (n - 1) + gamma + 1 : gamma + 1;
         child[i] = make_int2(left, right);
         range[i] = make_int2(lo, hi);
+        size[i] = hi - lo + 1;
         parent[left] = i;
         parent[right] = i;
     }
@@ -108,49 +106,6 @@ struct BoxF {
 __device__ __forceinline__ float half_area(const BoxF& b) {
     const float dx = b.hi[0] - b.lo[0], dy = b.hi[1] - b.lo[1], dz = b.hi[2] - b.lo[2];
     return dx * dy + dy * dz + dz * dx;
-}
-
-// Boxes and SAH costs bottom-up.  cost = node_cost * A + cost(left) + cost(right) for an
-// interior node, tri_cost * count * A for a leaf; a subtree of at most max_leaf triangles
-// whose leaf cost is no higher becomes one leaf (collapse[p] = 1).
-__global__ void k_refit(const float* __restrict__ v, const uint32_t* __restrict__ order, int n,
-                        const int2* __restrict__ child, const int2* __restrict__ range, const int* __restrict__ parent,
-                        BoxF* box, float* cost, uint32_t* collapse, uint32_t* flag, int max_leaf, float cn, float ct) {
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        const float* t = v + 9 * (size_t)order[k];
-        BoxF b;
-        for (int a = 0; a < 3; a++) {
-            b.lo[a] = fminf(fminf(t[a], t[3 + a]), t[6 + a]);
-            b.hi[a] = fmaxf(fmaxf(t[a], t[3 + a]), t[6 + a]);
-        }
-        int node = (n - 1) + k;
-        box[node] = b;
-        cost[node] = ct * half_area(b);
-        __threadfence();
-        int p = parent[node];
-        while (p >= 0) {
-            // the first thread to arrive leaves; the second has both children's results
-            if (atomicAdd(&flag[p], 1u) == 0u) break;
-            __threadfence();
-            const int2 ch = child[p];
-            const BoxF l = box[ch.x], r = box[ch.y];
-            BoxF m;
-            for (int a = 0; a < 3; a++) {
-                m.lo[a] = fminf(l.lo[a], r.lo[a]);
-                m.hi[a] = fmaxf(l.hi[a], r.hi[a]);
-            }
-            const float area = half_area(m);
-            const float c_int = cn * area + cost[ch.x] + cost[ch.y];
-            const int2 rg = range[p];
-            const int cnt = rg.y - rg.x + 1;
-            const float c_leaf = cnt <= max_leaf ? ct * (float)cnt * area : 3.0e38f;
-            box[p] = m;
-            cost[p] = fminf(c_int, c_leaf);
-            collapse[p] = c_leaf <= c_int ? 1u : 0u;
-            __threadfence();
-            p = parent[p];
-        }
-    }
 }
 
 // Leaf k (node (n - 1) + k, triangle order[k] of the Morton order): box, SAH cost, one
@@ -172,162 +127,388 @@ __global__ void k_leaves(const float* __restrict__ v, const uint32_t* __restrict
     }
 }
 
-constexpr int kTreeletBlock = 64;
 constexpr int kTreeletMinTris = 8;
 
-__device__ __forceinline__ TreeletBox to_tb(const BoxF& b) {
-    TreeletBox t;
-    for (int a = 0; a < 3; a++) {
-        t.lo[a] = b.lo[a];
-        t.hi[a] = b.hi[a];
+// ---- tiers: passes over the tree without global counters -----------------------------------------
+// A bottom-up pass in which every leaf's thread climbs to the root (an atomic counter a node, the
+// second to arrive goes on) needs device-wide fences at every step, and with eight non-coherent L2s
+// those cost more than the work: 1.1 ms to refit 164,000 triangles, 4.3 ms a treelet sweep with one
+// thread a treelet besides.  Here the tree is cut by subtree size into tiers.  A tier's roots are
+// the maximal subtrees of at most `hi` triangles; one block takes a root and works on its nodes of
+// more than `lo` triangles alone: it lists them level by level from the root, then goes through the
+// levels (deepest first or last) with block barriers between.  Kernel boundaries order the tiers.
+// 164,000 triangles: a treelet sweep 4.3 -> 1.16 ms, the refit 1.1 -> 0.06 ms, the ranges 31 launches and
+// downloads -> 3 launches (bound: the chain of treelets up a path, ~12 us each).
+constexpr int kTiers = 3;
+constexpr int kTierHi[kTiers] = {256, 32768, 0x7fffffff};
+constexpr int kTierThreads[kTiers] = {256, 512, 1024};
+
+__device__ __forceinline__ int tier_of(int size) { return size <= kTierHi[0] ? 0 : size <= kTierHi[1] ? 1 : 2; }
+
+struct TierRoots {
+    int2* roots[kTiers];  // (node, start of its part of the node list)
+    uint32_t* count;      // [kTiers] roots, [kTiers] list words handed out
+};
+
+// Roots of every tier.  A subtree of s triangles holds fewer than s interior nodes, and a tier's roots are
+// disjoint, so a list of n words holds the nodes of all of them.
+__global__ void k_tier_roots(int n, const int* __restrict__ parent, const int* __restrict__ size, TierRoots t) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n - 1; i += gridDim.x * blockDim.x) {
+        const int s = size[i], k = tier_of(s), p = parent[i];
+        if (p >= 0 && tier_of(size[p]) == k) continue;
+        const uint32_t j = atomicAdd(&t.count[k], 1u), at = atomicAdd(&t.count[kTiers + k], (uint32_t)s);
+        t.roots[k][j] = make_int2(i, (int)at);
     }
-    return t;
 }
 
-// Re-optimises the treelet under p (p's box, size and cost are current, as are those of every
-// node below it).  Its leaves: p's children, then repeatedly the largest-area interior leaf
-// replaced by its two children, up to kTreeletLeaves; its interior nodes are p and the nodes
-// so replaced, and they are reused for the new topology.
-template <class Cost>
+// The whole block: nodes of more than `lo` triangles under `root`, level by level, in list; returns the
+// number of levels (level l is list[level[l] .. level[l + 1])).  visit(x) runs once per listed node, after
+// the level above was visited.
+template <class Visit>
+__device__ int tier_levels(int root, int lo, int n, const int2* child, const int* size, int* list, int* level, uint32_t* sh,
+                           Visit visit) {
+    if (threadIdx.x == 0) {
+        list[0] = root;
+        level[0] = 0;
+        sh[0] = 1;
+    }
+    __syncthreads();
+    uint32_t b = 0, e = 1;
+    int nl = 0;
+    while (b < e) {
+        for (uint32_t i = b + threadIdx.x; i < e; i += blockDim.x) {
+            const int x = list[i];
+            const int2 c = child[x];
+            visit(x, c);
+            if (c.x < n - 1 && size[c.x] > lo) list[atomicAdd(&sh[0], 1u)] = c.x;
+            if (c.y < n - 1 && size[c.y] > lo) list[atomicAdd(&sh[0], 1u)] = c.y;
+        }
+        __syncthreads();
+        b = e;
+        e = sh[0];
+        nl++;
+        if (threadIdx.x == 0) level[nl] = (int)b;
+        __syncthreads();
+    }
+    return nl;
+}
+
+// One wave's treelet in LDS.
+struct TreeletWave {
+    float cost[kTreeletSubsets];  // cheapest cost of each subset of the treelet's leaves
+    float area[kTreeletSubsets];
+    TreeletBox box[kTreeletLeaves];
+    int leaf[kTreeletLeaves], lsize[kTreeletLeaves];
+    float lcost[kTreeletLeaves];
+    int inner[kTreeletLeaves - 1];
+    // the new topology: interior nodes in top-down order
+    uint32_t set[kTreeletLeaves - 1];
+    int node[kTreeletLeaves - 1], kid[kTreeletLeaves - 1][2], nsize[kTreeletLeaves - 1];
+    float ncost[kTreeletLeaves - 1];
+};
+
+// j's bits moved to the set bits of mask, lowest first.
+__device__ __forceinline__ uint32_t deposit(uint32_t j, uint32_t mask) {
+    uint32_t r = 0;
+    while (mask) {
+        const uint32_t b = mask & (0u - mask);
+        if (j & 1u) r |= b;
+        j >>= 1;
+        mask ^= b;
+    }
+    return r;
+}
+
+// The whole wave re-optimises the treelet under p (p's box, size and cost are current, as are those of
+// every node below it).  Its leaves: p's children, then repeatedly the largest-area interior leaf
+// replaced by its two children, up to kTreeletLeaves; its interior nodes are p and the nodes so
+// replaced, and they are reused for the new topology.  Lane l holds leaf l while it grows; the dynamic
+// programme runs a subset a lane (sizes 2 to 5), then the splits of a subset over lanes.
 __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* box, float* cost, int* size, float cn,
-                                 Cost C) {
-    int leaf[kTreeletLeaves], inner[kTreeletLeaves - 1];
-    int nl = 2, ni = 1;
-    inner[0] = p;
+                                 TreeletWave& w) {
+    const int lane = __lane_id();
     const int2 c0 = child[p];
-    leaf[0] = c0.x;
-    leaf[1] = c0.y;
+    int id = lane == 0 ? c0.x : c0.y;
+    BoxF bx = {{0, 0, 0}, {0, 0, 0}};
+    float lc = 0.0f, area = -1.0f;
+    int2 kids = make_int2(0, 0);
+    int sz = 0;
+    auto load = [&]() {
+        bx = box[id];
+        lc = cost[id];
+        sz = size[id];
+        if (id < n - 1) {
+            kids = child[id];
+            area = half_area(bx);
+        } else {
+            area = -1.0f;
+        }
+    };
+    if (lane < 2) load();
+    int nl = 2, ni = 1;
+    if (lane == 0) w.inner[0] = p;
     while (nl < kTreeletLeaves) {
-        int best = -1;
-        float ba = -1.0f;
-        for (int i = 0; i < nl; i++)
-            if (leaf[i] < n - 1) {
-                const float a = half_area(box[leaf[i]]);
-                if (a > ba) {
-                    ba = a;
-                    best = i;
-                }
+        // the largest interior leaf, the first of equals
+        float a = area;
+        int best = lane;
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) {
+            const float oa = __shfl_xor(a, o);
+            const int ob = __shfl_xor(best, o);
+            if (oa > a || (oa == a && ob < best)) {
+                a = oa;
+                best = ob;
             }
-        if (best < 0) break;
-        const int x = leaf[best];
-        inner[ni++] = x;
-        const int2 cx = child[x];
-        leaf[best] = cx.x;
-        leaf[nl++] = cx.y;
+        }
+        a = __shfl(a, 0);
+        best = __shfl(best, 0);
+        if (!(a > -1.0f)) break;
+        const int x = __shfl(id, best), cx = __shfl(kids.x, best), cy = __shfl(kids.y, best);
+        if (lane == 0) w.inner[ni] = x;
+        ni++;
+        if (lane == best || lane == nl) {
+            id = lane == best ? cx : cy;
+            load();
+        }
+        nl++;
     }
     if (nl < 3) return;  // two leaves have one topology
-    TreeletBox tb[kTreeletLeaves];
-    float lc[kTreeletLeaves];
-    for (int i = 0; i < nl; i++) {
-        tb[i] = to_tb(box[leaf[i]]);
-        lc[i] = cost[leaf[i]];
+    if (lane < nl) {
+        TreeletBox t;
+        for (int a = 0; a < 3; a++) {
+            t.lo[a] = bx.lo[a];
+            t.hi[a] = bx.hi[a];
+        }
+        w.box[lane] = t;
+        w.leaf[lane] = id;
+        w.lsize[lane] = sz;
+        w.lcost[lane] = lc;
+        w.cost[1u << lane] = lc;
     }
-    treelet_costs(tb, lc, nl, cn, C);
+    wave_lds_sync();
     const uint32_t full = (1u << nl) - 1u;
-    if (!(C(full) < cost[p] * (1.0f - 1e-6f))) return;
-    // new topology top-down (each split's parts go to a leaf or the next spare interior node),
-    // then boxes, sizes and costs of the interior nodes, children before parents
-    uint32_t set[kTreeletLeaves - 1];
-    int node[kTreeletLeaves - 1];
+    for (uint32_t s = (uint32_t)lane; s <= full; s += 64u) {
+        TreeletBox u = {{3.0e38f, 3.0e38f, 3.0e38f}, {-3.0e38f, -3.0e38f, -3.0e38f}};
+        for (int i = 0; i < nl; i++)
+            if (s >> i & 1u) treelet_union(u, w.box[i]);
+        w.area[s] = treelet_half_area(u);
+    }
+    wave_lds_sync();
+    for (int k = 2; k <= min(nl, 5); k++) {
+        for (uint32_t s = (uint32_t)lane; s <= full; s += 64u)
+            if (__popc(s) == k) {
+                const uint32_t low = s & (0u - s), rest = s ^ low;
+                float best = 3.0e38f;
+                for (uint32_t q = (rest - 1u) & rest;; q = (q - 1u) & rest) {
+                    best = fminf(best, w.cost[low | q] + w.cost[s ^ (low | q)]);
+                    if (q == 0u) break;
+                }
+                w.cost[s] = cn * w.area[s] + best;
+            }
+        wave_lds_sync();
+    }
+    // a subset of k leaves has 2^(k-1) - 1 splits: one a lane
+    auto split_cost = [&](uint32_t s, uint32_t j, uint32_t& q) {
+        const uint32_t low = s & (0u - s), rest = s ^ low;
+        q = deposit(j, rest);
+        const bool valid = j < (1u << (__popc(s) - 1)) - 1u;
+        return valid ? w.cost[low | q] + w.cost[s ^ (low | q)] : 3.0e38f;
+    };
+    for (int k = 6; k <= nl; k++) {
+        // nl = 6: the full set; nl = 7: the seven subsets of six, two at a time, then the full set
+        const int count = nl - k == 1 ? kTreeletLeaves : 1, half = lane >> 5;
+        for (int i = 0; i < count; i += k == 6 ? 2 : 1) {
+            const int drop = i + (k == 6 ? half : 0);
+            const uint32_t s = count == 1 ? full : full ^ (1u << min(drop, kTreeletLeaves - 1));
+            uint32_t q;
+            float best = split_cost(s, k == 6 ? (uint32_t)lane & 31u : (uint32_t)lane, q);
+            for (int o = k == 6 ? 16 : 32; o > 0; o >>= 1) best = fminf(best, __shfl_xor(best, o));
+            if ((k == 6 ? (lane & 31) : lane) == 0 && drop < kTreeletLeaves) w.cost[s] = cn * w.area[s] + best;
+        }
+        wave_lds_sync();
+    }
+    if (!(w.cost[full] < cost[p] * (1.0f - 1e-6f))) return;
+    // New topology top-down: each split's parts (the one treelet_split picks: the cheapest, of equals the
+    // one whose part without the lowest leaf is numerically largest) go to a leaf or the next spare node.
     int head = 0, tail = 1, next = 1;
-    set[0] = full;
-    node[0] = p;
+    if (lane == 0) {
+        w.set[0] = full;
+        w.node[0] = p;
+    }
+    wave_lds_sync();
     while (head < tail) {
-        const uint32_t s = set[head];
-        const int x = node[head];
-        head++;
-        const uint32_t a = treelet_split(s, C);
-        const uint32_t parts[2] = {a, s ^ a};
+        const uint32_t s = w.set[head];
+        const int x = w.node[head];
+        uint32_t q;
+        float c = split_cost(s, (uint32_t)lane, q);
+        int from = lane;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float oc = __shfl_xor(c, o);
+            const int of = __shfl_xor(from, o);
+            if (oc < c || (oc == c && of > from)) {
+                c = oc;
+                from = of;
+            }
+        }
+        const uint32_t low = s & (0u - s);
+        const uint32_t a = low | (uint32_t)__shfl((int)q, from);
         int ids[2];
         for (int k = 0; k < 2; k++) {
-            const uint32_t q = parts[k];
-            if ((q & (q - 1u)) == 0u) {
-                ids[k] = leaf[__ffs(q) - 1];
+            const uint32_t part = k == 0 ? a : s ^ a;
+            if ((part & (part - 1u)) == 0u) {
+                ids[k] = w.leaf[__ffs(part) - 1];
             } else {
-                ids[k] = inner[next++];
-                set[tail] = q;
-                node[tail] = ids[k];
+                ids[k] = w.inner[next++];
+                if (lane == 0) {
+                    w.set[tail] = part;
+                    w.node[tail] = ids[k];
+                }
                 tail++;
             }
-            parent[ids[k]] = x;
         }
-        child[x] = make_int2(ids[0], ids[1]);
+        if (lane == 0) {
+            w.kid[head][0] = (int)a;
+            w.kid[head][1] = (int)(s ^ a);
+            child[x] = make_int2(ids[0], ids[1]);
+            parent[ids[0]] = x;
+            parent[ids[1]] = x;
+        }
+        head++;
+        wave_lds_sync();
     }
+    // boxes, sizes and costs of the interior nodes, children before parents
     for (int j = tail - 1; j >= 0; j--) {
-        const int x = node[j];
-        const int2 ch = child[x];
-        const BoxF l = box[ch.x], r = box[ch.y];
-        BoxF m;
-        for (int a = 0; a < 3; a++) {
-            m.lo[a] = fminf(l.lo[a], r.lo[a]);
-            m.hi[a] = fmaxf(l.hi[a], r.hi[a]);
-        }
-        box[x] = m;
-        size[x] = size[ch.x] + size[ch.y];
-        cost[x] = cn * half_area(m) + cost[ch.x] + cost[ch.y];
-    }
-}
-
-// One bottom-up sweep: the second thread to reach a node (one atomic counter per node, as in
-// k_refit) has both subtrees final, refits the node and re-optimises its treelet.  Every
-// node a treelet touches lies under its root, whose subtrees are finished; the fence after
-// the counter makes the other subtree's writes visible.  Costs are the plain binary SAH
-// (the leaf collapse is decided after restructuring).
-__global__ __launch_bounds__(kTreeletBlock) void k_treelet(int n, int2* child, int* parent, BoxF* box, float* cost,
-                                                          int* size, uint32_t* flag, float cn) {
-    __shared__ float dp[kTreeletSubsets * kTreeletBlock];  // per thread one column of subset costs
-    float* col = dp + threadIdx.x;
-    auto C = [col](uint32_t s) -> float& { return col[s * kTreeletBlock]; };
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        int p = parent[(n - 1) + k];
-        while (p >= 0) {
-            if (atomicAdd(&flag[p], 1u) == 0u) break;
-            __threadfence();
-            const int2 ch = child[p];
-            const BoxF l = box[ch.x], r = box[ch.y];
-            BoxF m;
-            for (int a = 0; a < 3; a++) {
-                m.lo[a] = fminf(l.lo[a], r.lo[a]);
-                m.hi[a] = fmaxf(l.hi[a], r.hi[a]);
-            }
-            box[p] = m;
-            size[p] = size[ch.x] + size[ch.y];
-            cost[p] = cn * half_area(m) + cost[ch.x] + cost[ch.y];
-            if (size[p] >= kTreeletMinTris) treelet_optimise(p, n, child, parent, box, cost, size, cn, C);
-            __threadfence();
-            p = parent[p];
-        }
-    }
-}
-
-// One level of the top-down pass: each frontier node hands its range start to its children
-// (left first) and appends its interior children to the next frontier (one atomic per wave).
-__global__ void k_ranges_level(const int* __restrict__ frontier, uint32_t nf, const int2* __restrict__ child,
-                               const int* __restrict__ size, int2* range, int* next, uint32_t* next_count, int n) {
-    for (uint32_t base = blockIdx.x * blockDim.x; base < nf; base += gridDim.x * blockDim.x) {
-        const uint32_t i = base + threadIdx.x;
-        int c[2] = {-1, -1};
-        if (i < nf) {
-            const int x = frontier[i];
-            const int2 ch = child[x];
-            const int s = range[x].x;
-            const int sl = size[ch.x], sr = size[ch.y];
-            range[ch.x] = make_int2(s, s + sl - 1);
-            range[ch.y] = make_int2(s + sl, s + sl + sr - 1);
-            c[0] = ch.x < n - 1 ? ch.x : -1;
-            c[1] = ch.y < n - 1 ? ch.y : -1;
-        }
+        const uint32_t s = w.set[j];
+        const int x = w.node[j];
+        float kc[2];
+        int total = 0;
         for (int k = 0; k < 2; k++) {
-            const bool push = c[k] >= 0;
-            const uint64_t m = __ballot(push);
-            if (m == 0) continue;
-            const int lane = __lane_id();
-            const int leader = __ffsll((unsigned long long)m) - 1;
-            uint32_t b = 0;
-            if (lane == leader) b = atomicAdd(next_count, (uint32_t)__popcll(m));
-            b = __shfl(b, leader);
-            if (push) next[b + __popcll(m & ((1ull << lane) - 1ull))] = c[k];
+            const uint32_t part = (uint32_t)w.kid[j][k];
+            if ((part & (part - 1u)) == 0u) {
+                kc[k] = w.lcost[__ffs(part) - 1];
+                total += w.lsize[__ffs(part) - 1];
+            } else {
+                int at = j + 1;
+                while (w.set[at] != part) at++;
+                kc[k] = w.ncost[at];
+                total += w.nsize[at];
+            }
         }
+        const float c = cn * w.area[s] + kc[0] + kc[1];
+        if (lane < 6) {
+            const int a = lane % 3;
+            float v = lane < 3 ? 3.0e38f : -3.0e38f;
+            for (int i = 0; i < nl; i++)
+                if (s >> i & 1u) v = lane < 3 ? fminf(v, w.box[i].lo[a]) : fmaxf(v, w.box[i].hi[a]);
+            (lane < 3 ? box[x].lo : box[x].hi)[a] = v;
+        }
+        if (lane == 0) {
+            size[x] = total;
+            cost[x] = c;
+            w.nsize[j] = total;
+            w.ncost[j] = c;
+        }
+        wave_lds_sync();
+    }
+}
+
+// One tier of a bottom-up treelet sweep: level by level from the deepest, every node is refitted (a
+// thread a node) and the treelets of the level's large nodes are re-optimised (a wave a treelet).
+// Every node a treelet touches lies under its root, whose subtrees are finished.  Costs are the plain
+// binary SAH (the leaf collapse is decided after restructuring).
+template <int T>
+__global__ __launch_bounds__(kTierThreads[T]) void k_treelet(int n, TierRoots t, int2* child, int* parent, BoxF* box,
+                                                            float* cost, int* size, int* list_all, int* level_all, float cn) {
+    __shared__ TreeletWave tw[kTierThreads[T] / 64];
+    __shared__ uint32_t sh[1];
+    constexpr int kLo = T == 0 ? 1 : kTierHi[T > 0 ? T - 1 : 0];
+    const uint32_t nr = t.count[T];
+    const int wv = threadIdx.x >> 6, nw = kTierThreads[T] / 64;
+    for (uint32_t r = blockIdx.x; r < nr; r += gridDim.x) {
+        const int2 root = t.roots[T][r];
+        int *list = list_all + root.y, *level = level_all + root.y;
+        const int levels = tier_levels(root.x, kLo, n, child, size, list, level, sh, [](int, int2) {});
+        for (int l = levels - 1; l >= 0; l--) {
+            const int b = level[l], e = level[l + 1];
+            for (int i = b + (int)threadIdx.x; i < e; i += kTierThreads[T]) {
+                const int p = list[i];
+                const int2 ch = child[p];
+                const BoxF x = box[ch.x], y = box[ch.y];
+                BoxF m;
+                for (int a = 0; a < 3; a++) {
+                    m.lo[a] = fminf(x.lo[a], y.lo[a]);
+                    m.hi[a] = fmaxf(x.hi[a], y.hi[a]);
+                }
+                box[p] = m;
+                size[p] = size[ch.x] + size[ch.y];
+                cost[p] = cn * half_area(m) + cost[ch.x] + cost[ch.y];
+            }
+            __syncthreads();
+            for (int i = b + wv; i < e; i += nw) {
+                const int p = list[i];
+                if (size[p] >= kTreeletMinTris) treelet_optimise(p, n, child, parent, box, cost, size, cn, tw[wv]);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// One tier of the final bottom-up pass: boxes and SAH costs.  cost = node_cost * A + cost(left) +
+// cost(right) for an interior node, tri_cost * count * A for a leaf; a subtree of at most max_leaf
+// triangles whose leaf cost is no higher becomes one leaf (collapse[p] = 1).
+template <int T>
+__global__ __launch_bounds__(kTierThreads[T]) void k_refit(int n, TierRoots t, const int2* __restrict__ child, BoxF* box,
+                                                          float* cost, const int* __restrict__ size, uint32_t* collapse,
+                                                          int* list_all, int* level_all, int max_leaf, float cn, float ct) {
+    __shared__ uint32_t sh[1];
+    constexpr int kLo = T == 0 ? 1 : kTierHi[T > 0 ? T - 1 : 0];
+    const uint32_t nr = t.count[T];
+    for (uint32_t r = blockIdx.x; r < nr; r += gridDim.x) {
+        const int2 root = t.roots[T][r];
+        int *list = list_all + root.y, *level = level_all + root.y;
+        const int levels = tier_levels(root.x, kLo, n, child, size, list, level, sh, [](int, int2) {});
+        for (int l = levels - 1; l >= 0; l--) {
+            const int b = level[l], e = level[l + 1];
+            for (int i = b + (int)threadIdx.x; i < e; i += kTierThreads[T]) {
+                const int p = list[i];
+                const int2 ch = child[p];
+                const BoxF x = box[ch.x], y = box[ch.y];
+                BoxF m;
+                for (int a = 0; a < 3; a++) {
+                    m.lo[a] = fminf(x.lo[a], y.lo[a]);
+                    m.hi[a] = fmaxf(x.hi[a], y.hi[a]);
+                }
+                const float area = half_area(m);
+                const float c_int = cn * area + cost[ch.x] + cost[ch.y];
+                const int cnt = size[p];
+                const float c_leaf = cnt <= max_leaf ? ct * (float)cnt * area : 3.0e38f;
+                box[p] = m;
+                cost[p] = fminf(c_int, c_leaf);
+                collapse[p] = c_leaf <= c_int ? 1u : 0u;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// One tier of the top-down pass (the upper tiers first): each node hands its range start to its
+// children, left first.
+template <int T>
+__global__ __launch_bounds__(kTierThreads[T]) void k_ranges(int n, TierRoots t, const int2* __restrict__ child,
+                                                           const int* __restrict__ size, int2* range, int* list_all,
+                                                           int* level_all) {
+    __shared__ uint32_t sh[1];
+    constexpr int kLo = T == 0 ? 1 : kTierHi[T > 0 ? T - 1 : 0];
+    const uint32_t nr = t.count[T];
+    for (uint32_t r = blockIdx.x; r < nr; r += gridDim.x) {
+        const int2 root = t.roots[T][r];
+        tier_levels(root.x, kLo, n, child, size, list_all + root.y, level_all + root.y, sh, [&](int x, int2 c) {
+            const int s = range[x].x, sl = size[c.x], sr = size[c.y];
+            range[c.x] = make_int2(s, s + sl - 1);
+            range[c.y] = make_int2(s + sl, s + sl + sr - 1);
+        });
+        __syncthreads();
     }
 }
 
@@ -367,14 +548,24 @@ __global__ void k_emit(const int2* __restrict__ child, const int2* __restrict__ 
 }
 
 struct Bufs {
-    DevBuf dv, codes, idx, codes_s, idx_s, tmp, child, range, parent, box, cost, collapse, flag, nodes, size, front[2],
-        front_n, order;
-    ~Bufs() {
-        for (DevBuf* b : {&dv, &codes, &idx, &codes_s, &idx_s, &tmp, &child, &range, &parent, &box, &cost, &collapse,
-                          &flag, &nodes, &size, &front[0], &front[1], &front_n, &order})
-            b->release();
-    }
+    DevBuf dv, codes, idx, codes_s, idx_s, tmp, child, range, parent, box, cost, collapse, nodes, size, roots[kTiers],
+        tier_n, list, level, order;
 };
+
+// The three kernels of a pass over the tiers, `up` from the small subtrees to the root or down.
+template <class Launch>
+int for_tiers(bool up, int64_t n, Launch launch) {
+    for (int k = 0; k < kTiers; k++) {
+        const int t = up ? k : kTiers - 1 - k;
+        if (t > 0 && n <= kTierHi[t - 1]) continue;  // no subtree is that large
+        // roots are taken in turn; the smallest tier has at most one root a triangle pair, in practice
+        // one per ~150 triangles
+        const int64_t want = t == 0 ? n / 64 + 1 : t == 1 ? n / kTierHi[0] + 1 : 1;
+        launch(t, dim3((unsigned)std::min<int64_t>(want, t == 0 ? 8192 : 1024)), dim3((unsigned)kTierThreads[t]));
+        SPK_CHECK_HIP(hipGetLastError());
+    }
+    return SPK_OK;
+}
 
 // Depth-first renumbering of the reachable nodes: the left child follows its parent,
 // and interior nodes inside collapsed subtrees are dropped.
@@ -435,7 +626,9 @@ int build_bvh_gpu(const float* verts, int64_t n, const BvhBuildOpts& opts, BvhRe
         (rc = B.size.alloc((size_t)(2 * n) * 4)) ||
         (rc = B.parent.alloc((size_t)(2 * n) * 4)) || (rc = B.box.alloc((size_t)(2 * n) * sizeof(BoxF))) ||
         (rc = B.cost.alloc((size_t)(2 * n) * 4)) || (rc = B.collapse.alloc((size_t)n * 4)) ||
-        (rc = B.flag.alloc((size_t)n * 4)) || (rc = B.nodes.alloc((size_t)(n - 1) * sizeof(BvhNodeHost))))
+        (rc = B.list.alloc((size_t)(n + 1) * 4)) || (rc = B.level.alloc((size_t)(n + 1) * 4)) ||
+        (rc = B.tier_n.alloc(2 * kTiers * 4)) || (rc = B.roots[0].alloc((size_t)n * 8)) ||
+        (rc = B.roots[1].alloc((size_t)(n / kTierHi[0] + 2) * 8)) || (rc = B.roots[2].alloc(64)) || (rc = B.nodes.alloc((size_t)(n - 1) * sizeof(BvhNodeHost))))
         return rc;
     const int blocks = (int)std::min<int64_t>((n + 255) / 256, 65536);
     hipLaunchKernelGGL(k_morton, dim3(blocks), dim3(256), 0, 0, B.dv.as<float>(), (uint32_t)n,
@@ -451,53 +644,60 @@ int build_bvh_gpu(const float* verts, int64_t n, const BvhBuildOpts& opts, BvhRe
                                             B.idx.as<uint32_t>(), B.idx_s.as<uint32_t>(), (uint32_t)N, 0u, 63u,
                                             (hipStream_t)0));
     hipLaunchKernelGGL(k_hierarchy, dim3(blocks), dim3(256), 0, 0, B.codes_s.as<uint64_t>(), N, B.child.as<int2>(),
-                       B.range.as<int2>(), B.parent.as<int>());
+                       B.range.as<int2>(), B.parent.as<int>(), B.size.as<int>());
     SPK_CHECK_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_leaves, dim3(blocks), dim3(256), 0, 0, B.dv.as<float>(), B.idx_s.as<uint32_t>(), N,
                        B.box.as<BoxF>(), B.cost.as<float>(), B.size.as<int>(), B.range.as<int2>(), opts.tri_cost);
     SPK_CHECK_HIP(hipGetLastError());
     const uint32_t* leaf_order = B.idx_s.as<uint32_t>();
+    TierRoots tr;
+    for (int t = 0; t < kTiers; t++) tr.roots[t] = B.roots[t].as<int2>();
+    tr.count = B.tier_n.as<uint32_t>();
+    int2* child = B.child.as<int2>();
+    int *parent = B.parent.as<int>(), *size = B.size.as<int>(), *list = B.list.as<int>(), *level = B.level.as<int>();
+    BoxF* box = B.box.as<BoxF>();
+    float* cost = B.cost.as<float>();
+    auto find_roots = [&]() -> int {
+        SPK_CHECK_HIP(hipMemsetAsync(B.tier_n.p, 0, 2 * kTiers * 4, 0));
+        hipLaunchKernelGGL(k_tier_roots, dim3(blocks), dim3(256), 0, 0, N, (const int*)parent, (const int*)size, tr);
+        SPK_CHECK_HIP(hipGetLastError());
+        return SPK_OK;
+    };
     if (opts.treelet_passes > 0 && n >= kTreeletMinTris) {
-        const int tblocks = (int)std::min<int64_t>((n + kTreeletBlock - 1) / kTreeletBlock, 65536);
+        const float cn = opts.node_cost;
         for (int pass = 0; pass < opts.treelet_passes; pass++) {
-            SPK_CHECK_HIP(hipMemset(B.flag.p, 0, (size_t)n * 4));
-            hipLaunchKernelGGL(k_treelet, dim3(tblocks), dim3(kTreeletBlock), 0, 0, N, B.child.as<int2>(),
-                               B.parent.as<int>(), B.box.as<BoxF>(), B.cost.as<float>(), B.size.as<int>(),
-                               B.flag.as<uint32_t>(), opts.node_cost);
-            SPK_CHECK_HIP(hipGetLastError());
+            if ((rc = find_roots())) return rc;
+            rc = for_tiers(true, n, [&](int t, dim3 g, dim3 th) {
+                if (t == 0) hipLaunchKernelGGL(k_treelet<0>, g, th, 0, 0, N, tr, child, parent, box, cost, size, list, level, cn);
+                else if (t == 1) hipLaunchKernelGGL(k_treelet<1>, g, th, 0, 0, N, tr, child, parent, box, cost, size, list, level, cn);
+                else hipLaunchKernelGGL(k_treelet<2>, g, th, 0, 0, N, tr, child, parent, box, cost, size, list, level, cn);
+            });
+            if (rc) return rc;
         }
-        // ranges top-down, one tree level per launch, from the root's [0, n - 1]
-        if ((rc = B.front[0].alloc((size_t)n * 4)) || (rc = B.front[1].alloc((size_t)n * 4)) ||
-            (rc = B.front_n.alloc(4)) || (rc = B.order.alloc((size_t)n * 4)))
-            return rc;
-        const int root = 0;
-        const int2 root_range = make_int2(0, N - 1);
-        SPK_CHECK_HIP(hipMemcpy(B.front[0].p, &root, 4, hipMemcpyHostToDevice));
-        SPK_CHECK_HIP(hipMemcpy(B.range.p, &root_range, 8, hipMemcpyHostToDevice));
-        uint32_t nf = 1;
-        for (int level = 0; nf > 0; level++) {
-            if (level > N) {
-                set_error("build_bvh_gpu: restructured tree deeper than its triangle count");
-                return SPK_ERR_STATE;
-            }
-            SPK_CHECK_HIP(hipMemset(B.front_n.p, 0, 4));
-            const int lb = (int)std::min<int64_t>((nf + 255) / 256, 65536);
-            hipLaunchKernelGGL(k_ranges_level, dim3(lb), dim3(256), 0, 0, B.front[level & 1].as<int>(), nf,
-                               B.child.as<int2>(), B.size.as<int>(), B.range.as<int2>(), B.front[(level + 1) & 1].as<int>(),
-                               B.front_n.as<uint32_t>(), N);
-            SPK_CHECK_HIP(hipGetLastError());
-            SPK_CHECK_HIP(hipMemcpy(&nf, B.front_n.p, 4, hipMemcpyDeviceToHost));
-        }
-        hipLaunchKernelGGL(k_leaf_order, dim3(blocks), dim3(256), 0, 0, B.idx_s.as<uint32_t>(), B.range.as<int2>(), N,
+        // ranges top-down from the root's [0, n - 1], which the Morton tree's root has already
+        if ((rc = B.order.alloc((size_t)n * 4)) || (rc = find_roots())) return rc;
+        int2* range = B.range.as<int2>();
+        rc = for_tiers(false, n, [&](int t, dim3 g, dim3 th) {
+            if (t == 0) hipLaunchKernelGGL(k_ranges<0>, g, th, 0, 0, N, tr, (const int2*)child, (const int*)size, range, list, level);
+            else if (t == 1) hipLaunchKernelGGL(k_ranges<1>, g, th, 0, 0, N, tr, (const int2*)child, (const int*)size, range, list, level);
+            else hipLaunchKernelGGL(k_ranges<2>, g, th, 0, 0, N, tr, (const int2*)child, (const int*)size, range, list, level);
+        });
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_leaf_order, dim3(blocks), dim3(256), 0, 0, B.idx_s.as<uint32_t>(), range, N,
                            B.order.as<uint32_t>());
         SPK_CHECK_HIP(hipGetLastError());
         leaf_order = B.order.as<uint32_t>();
+    } else if ((rc = find_roots())) {
+        return rc;
     }
-    SPK_CHECK_HIP(hipMemset(B.flag.p, 0, (size_t)n * 4));
-    hipLaunchKernelGGL(k_refit, dim3(blocks), dim3(256), 0, 0, B.dv.as<float>(), B.idx_s.as<uint32_t>(), N,
-                       B.child.as<int2>(), B.range.as<int2>(), B.parent.as<int>(), B.box.as<BoxF>(), B.cost.as<float>(),
-                       B.collapse.as<uint32_t>(), B.flag.as<uint32_t>(), opts.max_leaf, opts.node_cost, opts.tri_cost);
-    SPK_CHECK_HIP(hipGetLastError());
+    rc = for_tiers(true, n, [&](int t, dim3 g, dim3 th) {
+        uint32_t* col = B.collapse.as<uint32_t>();
+        const float cn = opts.node_cost, ct = opts.tri_cost;
+        if (t == 0) hipLaunchKernelGGL(k_refit<0>, g, th, 0, 0, N, tr, (const int2*)child, box, cost, (const int*)size, col, list, level, opts.max_leaf, cn, ct);
+        else if (t == 1) hipLaunchKernelGGL(k_refit<1>, g, th, 0, 0, N, tr, (const int2*)child, box, cost, (const int*)size, col, list, level, opts.max_leaf, cn, ct);
+        else hipLaunchKernelGGL(k_refit<2>, g, th, 0, 0, N, tr, (const int2*)child, box, cost, (const int*)size, col, list, level, opts.max_leaf, cn, ct);
+    });
+    if (rc) return rc;
     hipLaunchKernelGGL(k_emit, dim3(blocks), dim3(256), 0, 0, B.child.as<int2>(), B.range.as<int2>(), B.box.as<BoxF>(), N,
                        B.collapse.as<uint32_t>(), B.nodes.as<BvhNodeHost>());
     SPK_CHECK_HIP(hipGetLastError());
