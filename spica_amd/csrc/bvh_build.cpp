@@ -394,47 +394,7 @@ int collapse_bvh4(const std::vector<BvhNodeHost>& n2, std::vector<Bvh4NodeHost>&
 // to the plane itself.
 void quantize_bvh4(const std::vector<Bvh4NodeHost>& in, std::vector<Bvh4QNodeHost>& out) {
     out.resize(in.size());
-    for (size_t i = 0; i < in.size(); i++) {
-        const Bvh4NodeHost& h = in[i];
-        Bvh4QNodeHost& q = out[i];
-        memset(&q, 0, sizeof(q));
-        for (int c = 0; c < 4; c++) q.link[c] = h.link[c];
-        for (int a = 0; a < 3; a++) {
-            float lo = FLT_MAX, hi = -FLT_MAX;
-            for (int c = 0; c < 4; c++)
-                if (h.link[c] != kBvh4Empty) {
-                    lo = std::min(lo, h.lo[a][c]);
-                    hi = std::max(hi, h.hi[a][c]);
-                }
-            if (lo > hi) lo = hi = 0.0f;  // no children (never for a built tree)
-            if (flush_subnormal(lo) > lo) lo = -FLT_MIN;
-            float sc = (hi - lo) / 255.0f;
-            // raise the step until code 255 reaches hi; the increment doubles, so a nearly flat
-            // box far from the origin needs a few rounds, not one per ulp of the step
-            for (float add = std::nextafter(sc, FLT_MAX) - sc; decode_q(255.0f, sc, lo) < hi; add *= 2.0f) sc += add;
-            q.origin[a] = lo;
-            q.scale[a] = sc;
-            uint32_t wlo = 0, whi = 0;
-            for (int c = 0; c < 4; c++) {
-                int ql = 0, qh = 0;
-                if (h.link[c] != kBvh4Empty) {
-                    const float cl = h.lo[a][c], ch = h.hi[a][c];
-                    if (sc > 0.0f) {
-                        ql = std::min(255, std::max(0, (int)std::floor((cl - lo) / sc)));
-                        qh = std::min(255, std::max(0, (int)std::ceil((ch - lo) / sc)));
-                        while (ql > 0 && decode_q((float)ql, sc, lo) > cl) ql--;
-                        while (ql < 255 && decode_q((float)(ql + 1), sc, lo) <= cl) ql++;
-                        while (qh < 255 && decode_q((float)qh, sc, lo) < ch) qh++;
-                        while (qh > 0 && decode_q((float)(qh - 1), sc, lo) >= ch) qh--;
-                    }
-                }
-                wlo |= (uint32_t)ql << (8 * c);
-                whi |= (uint32_t)qh << (8 * c);
-            }
-            q.qlo[a] = wlo;
-            q.qhi[a] = whi;
-        }
-    }
+    for (size_t i = 0; i < in.size(); i++) out[i] = quantize_node(in[i]);
 }
 
 }  // namespace spk

@@ -436,48 +436,51 @@ int spk_scene_create_ex(const spk_scene_desc* d, const spk_scene_build_opts* bop
     BvhBuildOpts bo;
     bo.max_leaf = bop.max_leaf;
     bo.treelet_passes = bop.treelet_passes;
-    BvhResult bvh;
-    if (bop.builder == SPK_BVH_LBVH) {
+    // Quantised 4-wide nodes and leaf order on the device: built there, or built on the host and
+    // uploaded (a scene of one triangle or none has no tree to build on the device).
+    BvhDev bvh;
+    if (bop.builder == SPK_BVH_LBVH && n >= 2) {
         if ((rc = build_bvh_gpu(d->verts, n, bo, bvh))) return rc;
     } else {
-        bvh = build_bvh(d->verts, n, bo);
-    }
-    std::vector<Bvh4QNodeHost> nodes4;
-    int depth4 = 0;
-    {
+        if (bop.builder == SPK_BVH_LBVH && (bo.max_leaf < 1 || bo.max_leaf > kMaxLeafTris)) {
+            set_error("build_bvh_gpu: max_leaf %d outside [1, %d]", bo.max_leaf, kMaxLeafTris);
+            return SPK_ERR_INVALID;
+        }
+        const BvhResult host = build_bvh(d->verts, n, bo);
         std::vector<Bvh4NodeHost> wide;
-        depth4 = collapse_bvh4(bvh.nodes, wide);
+        std::vector<Bvh4QNodeHost> nodes4;
+        bvh.max_depth = collapse_bvh4(host.nodes, wide);
         quantize_bvh4(wide, nodes4);
+        bvh.num_nodes = (int64_t)nodes4.size();
+        bvh.num_leaves = host.num_leaves;
+        if ((rc = bvh.nodes.upload(nodes4.data(), nodes4.size() * sizeof(Bvh4QNodeHost))) ||
+            (rc = bvh.order.upload(host.order.data(), host.order.size() * 4)))
+            return rc;
     }
+    const int depth4 = bvh.max_depth;
     auto t1 = std::chrono::steady_clock::now();
 
-    // Leaf-ordered triangle data (FP64 set-up, FP32 storage).
-    std::vector<float4> tris((size_t)n * 3), tri_ng((size_t)n), tri_n;
-    std::vector<int2> tri_ids((size_t)n);
+    // Leaf-ordered triangle data, formed on the device.
     bool any_smooth = false;
-    std::vector<TriFrame> frames((size_t)n);
-    for (int64_t i = 0; i < n; i++) {
-        frames[(size_t)i] = tri_frame(d->verts + 9 * i, d->normals ? d->normals + 9 * i : nullptr);
-        any_smooth = any_smooth || frames[(size_t)i].smooth;
+    for (int64_t i = 0; d->normals && i < n && !any_smooth; i++)
+        any_smooth = tri_frame(d->verts + 9 * i, d->normals + 9 * i).smooth;
+    {
+        DevBuf normals, mat_ids, light_ids;
+        const size_t N = (size_t)n;
+        if ((!bvh.verts.p && (rc = bvh.verts.upload(d->verts, N * 36))) ||
+            (d->normals && (rc = normals.upload(d->normals, N * 36))) || (rc = mat_ids.upload(d->mat_ids, N * 4)) ||
+            (d->light_ids && (rc = light_ids.upload(d->light_ids, N * 4))) || (rc = s->tris.alloc(N * 48)) ||
+            (rc = s->tri_ng.alloc(N * 16)) || (rc = s->tri_ids.alloc(N * 8)) || (any_smooth && (rc = s->tri_n.alloc(N * 48))))
+            return rc;
+        if ((rc = launch_tri_records(bvh.verts.as<float>(), d->normals ? normals.as<float>() : nullptr,
+                                     bvh.order.as<uint32_t>(), mat_ids.as<int32_t>(),
+                                     d->light_ids ? light_ids.as<int32_t>() : nullptr, n, s->tris.as<float4>(),
+                                     s->tri_ng.as<float4>(), s->tri_ids.as<int2>(),
+                                     any_smooth ? s->tri_n.as<float4>() : nullptr)))
+            return rc;
+        SPK_CHECK_HIP(hipStreamSynchronize(0));
     }
-    if (any_smooth) tri_n.resize((size_t)n * 3);
-    for (int64_t k = 0; k < n; k++) {
-        uint32_t prim = bvh.order[(size_t)k];
-        const TriFrame& f = frames[prim];
-        const float* v = d->verts + 9 * (size_t)prim;
-        float4 T0 = make_float4(v[0], v[1], v[2], 0.0f);
-        memcpy(&T0.w, &prim, 4);
-        tris[3 * k] = T0;
-        tris[3 * k + 1] = f4(dsub(f.p[1], f.p[0]), 0.0f);
-        tris[3 * k + 2] = f4(dsub(f.p[2], f.p[0]), 0.0f);
-        uint32_t mbits = (uint32_t)d->mat_ids[prim] | (f.smooth ? 0x80000000u : 0u);
-        float w;
-        memcpy(&w, &mbits, 4);
-        tri_ng[k] = f4(f.ng, w);
-        tri_ids[k] = make_int2((int)prim, d->light_ids ? d->light_ids[prim] : -1);
-        if (any_smooth)
-            for (int j = 0; j < 3; j++) tri_n[3 * k + j] = f4(f.n[j], 0.0f);
-    }
+    s->nodes = std::move(bvh.nodes);
 
     // Materials (bsdfs/*.cc setScatterFuncs).
     std::vector<MatDev> mats((size_t)std::max(1, d->num_materials));
@@ -549,7 +552,8 @@ int spk_scene_create_ex(const spk_scene_desc* d, const spk_scene_build_opts* bop
     // Area lights.
     std::vector<LightDev> lights((size_t)std::max(1, d->num_area_lights));
     for (int i = 0; i < d->num_area_lights; i++) {
-        const TriFrame& f = frames[(size_t)d->area_tri[i]];
+        const int64_t prim = d->area_tri[i];
+        const TriFrame f = tri_frame(d->verts + 9 * prim, d->normals ? d->normals + 9 * prim : nullptr);
         LightDev L;
         L.p0 = f4(f.p[0], (float)f.area);
         L.e1 = f4(dsub(f.p[1], f.p[0]), 0.0f);
@@ -648,11 +652,6 @@ int spk_scene_create_ex(const spk_scene_desc* d, const spk_scene_build_opts* bop
     }
 
     // Upload.
-    if ((rc = s->nodes.upload(nodes4.data(), nodes4.size() * sizeof(Bvh4QNodeHost)))) return rc;
-    if ((rc = s->tris.upload(tris.data(), tris.size() * sizeof(float4)))) return rc;
-    if ((rc = s->tri_ng.upload(tri_ng.data(), tri_ng.size() * sizeof(float4)))) return rc;
-    if ((rc = s->tri_ids.upload(tri_ids.data(), tri_ids.size() * sizeof(int2)))) return rc;
-    if (any_smooth && (rc = s->tri_n.upload(tri_n.data(), tri_n.size() * sizeof(float4)))) return rc;
     if ((rc = s->mats.upload(mats.data(), mats.size() * sizeof(MatDev)))) return rc;
     if ((rc = s->lights.upload(lights.data(), lights.size() * sizeof(LightDev)))) return rc;
     auto t2 = std::chrono::steady_clock::now();
@@ -683,17 +682,18 @@ int spk_scene_create_ex(const spk_scene_desc* d, const spk_scene_build_opts* bop
         s->lo[k] = 3.0e38f;
         s->hi[k] = -3.0e38f;
     }
-    for (int64_t i = 0; i < 9 * n; i++) {
-        s->lo[i % 3] = std::min(s->lo[i % 3], d->verts[i]);
-        s->hi[i % 3] = std::max(s->hi[i % 3], d->verts[i]);
-    }
+    for (int64_t i = 0; i < 3 * n; i++)
+        for (int k = 0; k < 3; k++) {
+            s->lo[k] = std::min(s->lo[k], d->verts[3 * i + k]);
+            s->hi[k] = std::max(s->hi[k], d->verts[3 * i + k]);
+        }
     if (n == 0)
         for (int k = 0; k < 3; k++) {
             s->lo[k] = 0.0f;
             s->hi[k] = 1.0f;
         }
     s->stats.num_tris = n;
-    s->stats.num_nodes = (int64_t)nodes4.size();
+    s->stats.num_nodes = bvh.num_nodes;
     s->stats.num_leaves = bvh.num_leaves;
     s->stats.max_depth = depth4;
     s->stats.num_lights = sd.num_lights;

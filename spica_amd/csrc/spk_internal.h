@@ -73,9 +73,9 @@ int collapse_bvh4(const std::vector<BvhNodeHost>& nodes2, std::vector<Bvh4NodeHo
 //
 // The traversal kernels flush single-precision subnormals (inputs and results, sign kept),
 // so the host decodes the way they do.
-inline float flush_subnormal(float x) { return std::fabs(x) < FLT_MIN ? std::copysign(0.0f, x) : x; }
-inline float decode_q(float q, float scale, float origin) {
-    return flush_subnormal(std::fmaf(q, flush_subnormal(scale), flush_subnormal(origin)));
+__host__ __device__ inline float flush_subnormal(float x) { return fabsf(x) < FLT_MIN ? copysignf(0.0f, x) : x; }
+__host__ __device__ inline float decode_q(float q, float scale, float origin) {
+    return flush_subnormal(fmaf(q, flush_subnormal(scale), flush_subnormal(origin)));
 }
 struct Bvh4QNodeHost {
     float origin[3];
@@ -85,10 +85,50 @@ struct Bvh4QNodeHost {
     int32_t link[4];
 };
 static_assert(sizeof(Bvh4QNodeHost) == 64, "quantised 4-wide node is 64 bytes");
+// One node, by the same code on the host and on the device (float division and fmaf are correctly
+// rounded on both; files that include this for device code keep IEEE division and subnormals).
+__host__ __device__ inline Bvh4QNodeHost quantize_node(const Bvh4NodeHost& h) {
+    Bvh4QNodeHost q;
+    for (int c = 0; c < 4; c++) q.link[c] = h.link[c];
+    for (int a = 0; a < 3; a++) {
+        float lo = FLT_MAX, hi = -FLT_MAX;
+        for (int c = 0; c < 4; c++)
+            if (h.link[c] != kBvh4Empty) {
+                lo = fminf(lo, h.lo[a][c]);
+                hi = fmaxf(hi, h.hi[a][c]);
+            }
+        if (lo > hi) lo = hi = 0.0f;  // no children (never for a built tree)
+        if (flush_subnormal(lo) > lo) lo = -FLT_MIN;
+        float sc = (hi - lo) / 255.0f;
+        // raise the step until code 255 reaches hi; the increment doubles, so a nearly flat
+        // box far from the origin needs a few rounds, not one per ulp of the step
+        for (float add = nextafterf(sc, FLT_MAX) - sc; decode_q(255.0f, sc, lo) < hi; add *= 2.0f) sc += add;
+        q.origin[a] = lo;
+        q.scale[a] = sc;
+        uint32_t wlo = 0, whi = 0;
+        for (int c = 0; c < 4; c++) {
+            int ql = 0, qh = 0;
+            if (h.link[c] != kBvh4Empty) {
+                const float cl = h.lo[a][c], ch = h.hi[a][c];
+                if (sc > 0.0f) {
+                    const float fl = floorf((cl - lo) / sc), fh = ceilf((ch - lo) / sc);
+                    ql = (int)fminf(255.0f, fmaxf(0.0f, fl));
+                    qh = (int)fminf(255.0f, fmaxf(0.0f, fh));
+                    while (ql > 0 && decode_q((float)ql, sc, lo) > cl) ql--;
+                    while (ql < 255 && decode_q((float)(ql + 1), sc, lo) <= cl) ql++;
+                    while (qh < 255 && decode_q((float)qh, sc, lo) < ch) qh++;
+                    while (qh > 0 && decode_q((float)(qh - 1), sc, lo) >= ch) qh--;
+                }
+            }
+            wlo |= (uint32_t)ql << (8 * c);
+            whi |= (uint32_t)qh << (8 * c);
+        }
+        q.qlo[a] = wlo;
+        q.qhi[a] = whi;
+    }
+    return q;
+}
 void quantize_bvh4(const std::vector<Bvh4NodeHost>& in, std::vector<Bvh4QNodeHost>& out);
-// Linear BVH on the device (Morton order, radix tree, bottom-up boxes); same node format.
-int build_bvh_gpu(const float* verts, int64_t n, const BvhBuildOpts& opts, BvhResult& res);
-
 // ---- device buffers -----------------------------------------------------------
 // One device allocation, freed when the owner goes out of scope (or on release()), so early
 // error returns and temporaries do not leak.  Not copyable; moving hands the allocation over.
@@ -120,6 +160,20 @@ struct DevBuf {
     template <class T>
     T* as() const { return reinterpret_cast<T*>(p); }
 };
+
+// Linear BVH built on the device (Morton order, radix tree, treelets, 4-wide collapse): the quantised
+// nodes, the leaf order and the vertices stay there.  At least two triangles.
+struct BvhDev {
+    DevBuf nodes, order, verts;
+    int64_t num_nodes = 0, num_leaves = 0;
+    int max_depth = 0;
+};
+int build_bvh_gpu(const float* verts, int64_t n, const BvhBuildOpts& opts, BvhDev& res);
+
+// ---- scene records (spk_scene.hip) ------------------------------------------------
+// Leaf-ordered triangle data from device arrays (normals, light_ids and tri_n may be null).
+int launch_tri_records(const float* verts, const float* normals, const uint32_t* order, const int32_t* mat_ids,
+                       const int32_t* light_ids, int64_t n, float4* tris, float4* tri_ng, int2* tri_ids, float4* tri_n);
 
 // ---- kernel launchers (spk_kernels.hip) -----------------------------------------
 struct TraceBufs {
