@@ -162,8 +162,8 @@ constexpr int kTreeletMinTris = 8;
 // the maximal subtrees of at most `hi` triangles; one block takes a root and works on its nodes of
 // more than `lo` triangles alone: it lists them level by level from the root, then goes through the
 // levels (deepest first or last) with block barriers between.  Kernel boundaries order the tiers.
-// 164,000 triangles: a treelet sweep 4.3 -> 1.16 ms, the refit 1.1 -> 0.06 ms, the ranges 31 launches and
-// downloads -> 3 launches (bound: the chain of treelets up a path, ~12 us each).
+// 164,000 triangles: a treelet sweep 4.3 -> 0.80 ms, the refit 1.1 -> 0.06 ms, the ranges 31 launches and
+// downloads -> 3 launches (bound: the chain of treelets up a path, ~8 us each).
 constexpr int kTiers = 3;
 constexpr int kTierHi[kTiers] = {256, 32768, 0x7fffffff};
 constexpr int kTierThreads[kTiers] = {256, 512, 1024};
@@ -223,13 +223,6 @@ struct TreeletWave {
     float cost[kTreeletSubsets];  // cheapest cost of each subset of the treelet's leaves
     float area[kTreeletSubsets];
     TreeletBox box[kTreeletLeaves];
-    int leaf[kTreeletLeaves], lsize[kTreeletLeaves];
-    float lcost[kTreeletLeaves];
-    int inner[kTreeletLeaves - 1];
-    // the new topology: interior nodes in top-down order
-    uint32_t set[kTreeletLeaves - 1];
-    int node[kTreeletLeaves - 1], kid[kTreeletLeaves - 1][2], nsize[kTreeletLeaves - 1];
-    float ncost[kTreeletLeaves - 1];
 };
 
 // j's bits moved to the set bits of mask, lowest first.
@@ -244,11 +237,40 @@ __device__ __forceinline__ uint32_t deposit(uint32_t j, uint32_t mask) {
     return r;
 }
 
+// Wave reductions by DPP: a step is one instruction of a few cycles, a shuffle through LDS about 60.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ float read_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+__device__ __forceinline__ float max8(float v) {  // over the 8 lanes of a group
+    v = fmaxf(v, dpp<kDppXor1>(v));
+    v = fmaxf(v, dpp<kDppXor2>(v));
+    return fmaxf(v, dpp<kDppHalfMirror>(v));
+}
+__device__ __forceinline__ float min16(float v) {  // over the 16 lanes of a row
+    v = fminf(v, dpp<kDppXor1>(v));
+    v = fminf(v, dpp<kDppXor2>(v));
+    v = fminf(v, dpp<kDppHalfMirror>(v));
+    return fminf(v, dpp<kDppMirror>(v));
+}
+__device__ __forceinline__ float min64(float v) {  // uniform
+    v = min16(v);
+    return fminf(fminf(read_lane(v, 0), read_lane(v, 16)), fminf(read_lane(v, 32), read_lane(v, 48)));
+}
+
 // The whole wave re-optimises the treelet under p (p's box, size and cost are current, as are those of
 // every node below it).  Its leaves: p's children, then repeatedly the largest-area interior leaf
 // replaced by its two children, up to kTreeletLeaves; its interior nodes are p and the nodes so
 // replaced, and they are reused for the new topology.  Lane l holds leaf l while it grows; the dynamic
-// programme runs a subset a lane (sizes 2 to 5), then the splits of a subset over lanes.
+// programme runs a subset a lane (sizes 2 to 5), then the splits of a subset over lanes.  One treelet
+// is a serial chain, so its steps are kept short: what one lane knows and all need is read with
+// v_readlane, minima are DPP steps and a ballot, and LDS holds only what is indexed by subset
+// (through shuffles and LDS throughout a sweep of 164,000 triangles took 1.16 ms, 0.80 so).
 __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* box, float* cost, int* size, float cn,
                                  TreeletWave& w) {
     const int lane = __lane_id();
@@ -271,25 +293,14 @@ __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* b
     };
     if (lane < 2) load();
     int nl = 2, ni = 1;
-    if (lane == 0) w.inner[0] = p;
+    int inner = p;  // lane i: the i-th interior node
     while (nl < kTreeletLeaves) {
-        // the largest interior leaf, the first of equals
-        float a = area;
-        int best = lane;
-#pragma unroll
-        for (int o = 4; o > 0; o >>= 1) {
-            const float oa = __shfl_xor(a, o);
-            const int ob = __shfl_xor(best, o);
-            if (oa > a || (oa == a && ob < best)) {
-                a = oa;
-                best = ob;
-            }
-        }
-        a = __shfl(a, 0);
-        best = __shfl(best, 0);
+        // the largest interior leaf, the first of equals (leaves sit in lanes 0 .. 6)
+        const float a = read_lane(max8(area), 0);
         if (!(a > -1.0f)) break;
-        const int x = __shfl(id, best), cx = __shfl(kids.x, best), cy = __shfl(kids.y, best);
-        if (lane == 0) w.inner[ni] = x;
+        const int best = __ffsll((long long)(__ballot(area == a) & 0xffull)) - 1;
+        const int x = read_lane(id, best), cx = read_lane(kids.x, best), cy = read_lane(kids.y, best);
+        if (lane == ni) inner = x;
         ni++;
         if (lane == best || lane == nl) {
             id = lane == best ? cx : cy;
@@ -305,9 +316,6 @@ __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* b
             t.hi[a] = bx.hi[a];
         }
         w.box[lane] = t;
-        w.leaf[lane] = id;
-        w.lsize[lane] = sz;
-        w.lcost[lane] = lc;
         w.cost[1u << lane] = lc;
     }
     wave_lds_sync();
@@ -347,7 +355,9 @@ __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* b
             const uint32_t s = count == 1 ? full : full ^ (1u << min(drop, kTreeletLeaves - 1));
             uint32_t q;
             float best = split_cost(s, k == 6 ? (uint32_t)lane & 31u : (uint32_t)lane, q);
-            for (int o = k == 6 ? 16 : 32; o > 0; o >>= 1) best = fminf(best, __shfl_xor(best, o));
+            best = min16(best);
+            const float lo = fminf(read_lane(best, 0), read_lane(best, 16)), hi = fminf(read_lane(best, 32), read_lane(best, 48));
+            best = k != 6 ? fminf(lo, hi) : half ? hi : lo;
             if ((k == 6 ? (lane & 31) : lane) == 0 && drop < kTreeletLeaves) w.cost[s] = cn * w.area[s] + best;
         }
         wave_lds_sync();
@@ -355,87 +365,77 @@ __device__ void treelet_optimise(int p, int n, int2* child, int* parent, BoxF* b
     if (!(w.cost[full] < cost[p] * (1.0f - 1e-6f))) return;
     // New topology top-down: each split's parts (the one treelet_split picks: the cheapest, of equals the
     // one whose part without the lowest leaf is numerically largest) go to a leaf or the next spare node.
+    // Node j of the new topology keeps its set, node and parts in lane j.
     int head = 0, tail = 1, next = 1;
-    if (lane == 0) {
-        w.set[0] = full;
-        w.node[0] = p;
-    }
-    wave_lds_sync();
+    int set = (int)full, node = p, kid0 = 0, kid1 = 0;  // a part: leaf l as -1 - l, or a later j
     while (head < tail) {
-        const uint32_t s = w.set[head];
-        const int x = w.node[head];
+        const uint32_t s = (uint32_t)read_lane(set, head);
+        const int x = read_lane(node, head);
         uint32_t q;
+        // (of the valid splits only, also where costs overflow)
+        const bool valid = (uint32_t)lane < (1u << (__popc(s) - 1)) - 1u;
         float c = split_cost(s, (uint32_t)lane, q);
-        int from = lane;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float oc = __shfl_xor(c, o);
-            const int of = __shfl_xor(from, o);
-            if (oc < c || (oc == c && of > from)) {
-                c = oc;
-                from = of;
-            }
-        }
-        const uint32_t low = s & (0u - s);
-        const uint32_t a = low | (uint32_t)__shfl((int)q, from);
-        int ids[2];
+        c = valid ? c : __builtin_inff();
+        const float m = min64(c);  // (every lane takes part)
+        const unsigned long long same = __ballot(valid && c == m);
+        const int from = same ? 63 - __clzll((long long)same) : 0;
+        const uint32_t a = (s & (0u - s)) | (uint32_t)read_lane((int)q, from);
+        int ids[2], kid[2];
         for (int k = 0; k < 2; k++) {
             const uint32_t part = k == 0 ? a : s ^ a;
             if ((part & (part - 1u)) == 0u) {
-                ids[k] = w.leaf[__ffs(part) - 1];
+                kid[k] = -__ffs(part);
+                ids[k] = read_lane(id, __ffs(part) - 1);
             } else {
-                ids[k] = w.inner[next++];
-                if (lane == 0) {
-                    w.set[tail] = part;
-                    w.node[tail] = ids[k];
+                ids[k] = read_lane(inner, next++);
+                if (lane == tail) {
+                    set = (int)part;
+                    node = ids[k];
                 }
-                tail++;
+                kid[k] = tail++;
             }
         }
+        if (lane == head) {
+            kid0 = kid[0];
+            kid1 = kid[1];
+        }
         if (lane == 0) {
-            w.kid[head][0] = (int)a;
-            w.kid[head][1] = (int)(s ^ a);
             child[x] = make_int2(ids[0], ids[1]);
             parent[ids[0]] = x;
             parent[ids[1]] = x;
         }
         head++;
-        wave_lds_sync();
     }
-    // boxes, sizes and costs of the interior nodes, children before parents
+    // boxes and sizes, a lane a plane or a node; costs, children before parents
+    const int j8 = lane >> 3, c6 = lane & 7;
+    const uint32_t s8 = (uint32_t)__shfl(set, j8);
+    const int x8 = __shfl(node, j8);
+    if (j8 < tail && c6 < 6) {
+        const int a = c6 % 3;
+        float v = c6 < 3 ? 3.0e38f : -3.0e38f;
+        for (int i = 0; i < nl; i++)
+            if (s8 >> i & 1u) v = c6 < 3 ? fminf(v, w.box[i].lo[a]) : fmaxf(v, w.box[i].hi[a]);
+        (c6 < 3 ? box[x8].lo : box[x8].hi)[a] = v;
+    }
+    int total = 0;
+    for (int i = 0; i < nl; i++) {
+        const int z = read_lane(sz, i);
+        total += (set >> i & 1) ? z : 0;
+    }
+    const float sa = w.area[set];
+    float nc = 0.0f;
     for (int j = tail - 1; j >= 0; j--) {
-        const uint32_t s = w.set[j];
-        const int x = w.node[j];
-        float kc[2];
-        int total = 0;
-        for (int k = 0; k < 2; k++) {
-            const uint32_t part = (uint32_t)w.kid[j][k];
-            if ((part & (part - 1u)) == 0u) {
-                kc[k] = w.lcost[__ffs(part) - 1];
-                total += w.lsize[__ffs(part) - 1];
-            } else {
-                int at = j + 1;
-                while (w.set[at] != part) at++;
-                kc[k] = w.ncost[at];
-                total += w.nsize[at];
-            }
-        }
-        const float c = cn * w.area[s] + kc[0] + kc[1];
-        if (lane < 6) {
-            const int a = lane % 3;
-            float v = lane < 3 ? 3.0e38f : -3.0e38f;
-            for (int i = 0; i < nl; i++)
-                if (s >> i & 1u) v = lane < 3 ? fminf(v, w.box[i].lo[a]) : fmaxf(v, w.box[i].hi[a]);
-            (lane < 3 ? box[x].lo : box[x].hi)[a] = v;
-        }
-        if (lane == 0) {
-            size[x] = total;
-            cost[x] = c;
-            w.nsize[j] = total;
-            w.ncost[j] = c;
-        }
-        wave_lds_sync();
+        const int k0 = read_lane(kid0, j), k1 = read_lane(kid1, j);
+        const float c0 = k0 < 0 ? read_lane(lc, -1 - k0) : read_lane(nc, k0);
+        const float c1 = k1 < 0 ? read_lane(lc, -1 - k1) : read_lane(nc, k1);
+        const float c = cn * read_lane(sa, j) + c0 + c1;
+        if (lane == j) nc = c;
     }
+    if (lane < tail) {
+        size[node] = total;
+        cost[node] = nc;
+    }
+    wave_lds_sync();
 }
 
 // One tier of a bottom-up treelet sweep: level by level from the deepest, every node is refitted (a
