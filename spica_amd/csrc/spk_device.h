@@ -2,7 +2,7 @@
 //
 // Everything the kernels read lives in HBM as arrays of 16-byte vectors so each
 // per-lane gather is one or more dwordx4 loads:
-//   BVH node      64 B  (four float4: both child boxes + child links)
+//   BVH node      64 B  (four child boxes, 8 bits a plane, and four links)
 //   triangle      48 B  (v0 | prim id, e1, e2) in leaf order
 //   shading rec   16+8 B (geometric normal | material, prim id / light id)
 #pragma once
