@@ -188,7 +188,15 @@ struct Counters {
 // wave's longest descent.  2 M closest hits, by eighths (0: wait for all): 0 351, 2 300, 3 288, 4 285, 5
 // 283, 6 289 us; 1080p x 32 frame 25.9, 23.5, 22.9, 22.7, 22.7, 22.8 ms; batch 15.5, 14.7, 14.6, 14.6, 14.9,
 // 15.2 ms.
-constexpr uint32_t kStayEighths = 4;
+//
+// A closest-hit ray culls boxes with the nearest hit it has tested so far, so how soon a postponed leaf is
+// tested decides which of two triangles a few ulp apart it reports (about 1 in 10^9 rays; box margins do
+// not cover a triangle's rounding there).  The render stages' closest-hit kernels therefore keep the
+// plain rule (kStayAll): a film of 66 M paths then repeats what it was, where the early rule moved one of
+// its samples in about one film of twelve (1080p x 32 frame 25.5 ms so, 22.9 ms with the early rule).
+// Any-hit rays cull with a fixed bound, so their answers do not depend on it; ray queries and the last
+// paths of a pass are few.
+constexpr uint32_t kStayEighths = 4, kStayAll = 0;
 
 // One lane's walk down the BVH.  Every traversal kernel uses it: start() a ray, then step() (the
 // whole wave together) until done().
@@ -319,7 +327,7 @@ struct Walker {
     // hand.  A lane holds one postponed leaf while it looks for the next, so a ray's triangles are
     // tested in its own depth-first order whatever the other lanes do.
     __device__ __forceinline__ void step(const float4* __restrict__ nodes, const float4* __restrict__ tris, bool any,
-                                         uint32_t busy, Counters& cnt) {
+                                         uint32_t stay, uint32_t busy, Counters& cnt) {
         while (node >= 0 && node != kSent) {
             visit(nodes, cnt);
             if (node < 0 && leaf == 0) {
@@ -327,7 +335,7 @@ struct Walker {
                 node = pop();
             }
             if (__all(leaf != 0)) break;
-            if ((uint32_t)__popcll(__ballot(1)) * 8u < busy * kStayEighths) break;
+            if ((uint32_t)__popcll(__ballot(1)) * 8u < busy * stay) break;
         }
         while (leaf < 0) {
             const uint32_t x = ~(uint32_t)leaf;
@@ -395,7 +403,7 @@ __device__ __forceinline__ const SceneDev& pick_scene(const SceneDev* p, const S
     else return s;
 }
 
-template <int BLOCK, int S, bool ANY, bool COUNT, bool BATCH, class Load, class Done>
+template <int BLOCK, int S, bool ANY, bool COUNT, bool BATCH, uint32_t STAY, class Load, class Done>
 __device__ __forceinline__ void traverse_stream(const SceneDev& sc0, const SceneDev* scenes, uint32_t count, Load load,
                                                 Done done, uint32_t* col, uint32_t* spill, Counters& cnt,
                                                 uint32_t chunk_log2 = 6) {
@@ -435,7 +443,7 @@ __device__ __forceinline__ void traverse_stream(const SceneDev& sc0, const Scene
         }
         const uint32_t busy = (uint32_t)__popcll(__ballot(active));
         if (busy == 0) break;
-        w.step(pick_scene<BATCH>(sc, sc0).nodes, pick_scene<BATCH>(sc, sc0).tris, ANY, busy, cnt);
+        w.step(pick_scene<BATCH>(sc, sc0).nodes, pick_scene<BATCH>(sc, sc0).tris, ANY, STAY, busy, cnt);
         if (active && w.done()) {
             done(idx, w.hit, w.tbest, w.hu, w.hv, pick_scene<BATCH>(sc, sc0));
             active = false;
@@ -467,7 +475,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void
             if (b.t_out) b.t_out[i] = k >= 0 ? t : -1.0f;
         }
     };
-    traverse_stream<BLOCK, S, ANY, false, false>(sc, nullptr, (uint32_t)b.n, load, done, col, spill, cnt, chunk_log2);
+    traverse_stream<BLOCK, S, ANY, false, false, kStayEighths>(sc, nullptr, (uint32_t)b.n, load, done, col, spill, cnt, chunk_log2);
 }
 
 // ---- pass bookkeeping -----------------------------------------------------------------------
@@ -729,7 +737,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(traversal
         rb.hit[i] = make_float4(t, u, v, __int_as_float(k));
         if (COUNT) rays++;
     };
-    traverse_stream<BLOCK, S, false, COUNT, BATCH>(sc, rb.scenes, count, load, done, col, spill, cnt);
+    traverse_stream<BLOCK, S, false, COUNT, BATCH, kStayAll>(sc, rb.scenes, count, load, done, col, spill, cnt);
     if (COUNT) {
         atomicAdd(&ps->count_nodes, (unsigned long long)cnt.nodes);
         atomicAdd(&ps->count_tris, (unsigned long long)cnt.tris);
@@ -1836,7 +1844,7 @@ __global__ __launch_bounds__(BLOCK) void k_shadow(SceneDev sc, RenderBufs rb, in
         }
         if (COUNT) rays++;
     };
-    traverse_stream<BLOCK, S, true, COUNT, BATCH>(sc, rb.scenes, count, load, done, col, spill, cnt);
+    traverse_stream<BLOCK, S, true, COUNT, BATCH, kStayEighths>(sc, rb.scenes, count, load, done, col, spill, cnt);
     if (COUNT) {
         atomicAdd(&ps->count_nodes_s, (unsigned long long)cnt.nodes);
         atomicAdd(&ps->count_tris_s, (unsigned long long)cnt.tris);
@@ -1881,7 +1889,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(BATCH ? 7
             rb.path_L[path] = make_float4(Lv.x + c.x * Le.x, Lv.y + c.y * Le.y, Lv.z + c.z * Le.z, Lv.w);
         }
     };
-    traverse_stream<BLOCK, S, false, false, BATCH>(sc, rb.scenes, count, load, done, col, spill, cnt);
+    traverse_stream<BLOCK, S, false, false, BATCH, kStayAll>(sc, rb.scenes, count, load, done, col, spill, cnt);
 }
 
 // ---- tail: the last paths of a pass, each to its end in one launch -----------------------------
@@ -1935,7 +1943,7 @@ __device__ __forceinline__ void traverse_pair(const SceneDev& sc, bool has1, boo
         }
         const uint32_t busy = (uint32_t)__popcll(__ballot(ray != 0));
         if (busy == 0) break;
-        w.step(sc.nodes, sc.tris, any, busy, cnt);
+        w.step(sc.nodes, sc.tris, any, kStayEighths, busy, cnt);
         if (ray != 0 && w.done()) {
             if (ray == 1) {
                 hit1 = make_float4(w.tbest, w.hu, w.hv, __int_as_float(w.hit));
