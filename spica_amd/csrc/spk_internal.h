@@ -94,8 +94,9 @@ __host__ __device__ inline Bvh4QNodeHost quantize_node(const Bvh4NodeHost& h) {
         float lo = FLT_MAX, hi = -FLT_MAX;
         for (int c = 0; c < 4; c++)
             if (h.link[c] != kBvh4Empty) {
-                lo = fminf(lo, h.lo[a][c]);
-                hi = fmaxf(hi, h.hi[a][c]);
+                // (comparisons: fminf and fmaxf are library calls on the host, 40 ms for 327,686 triangles)
+                lo = h.lo[a][c] < lo ? h.lo[a][c] : lo;
+                hi = h.hi[a][c] > hi ? h.hi[a][c] : hi;
             }
         if (lo > hi) lo = hi = 0.0f;  // no children (never for a built tree)
         if (flush_subnormal(lo) > lo) lo = -FLT_MIN;
@@ -112,8 +113,8 @@ __host__ __device__ inline Bvh4QNodeHost quantize_node(const Bvh4NodeHost& h) {
                 const float cl = h.lo[a][c], ch = h.hi[a][c];
                 if (sc > 0.0f) {
                     const float fl = floorf((cl - lo) / sc), fh = ceilf((ch - lo) / sc);
-                    ql = (int)fminf(255.0f, fmaxf(0.0f, fl));
-                    qh = (int)fminf(255.0f, fmaxf(0.0f, fh));
+                    ql = !(fl > 0.0f) ? 0 : fl < 255.0f ? (int)fl : 255;
+                    qh = !(fh > 0.0f) ? 0 : fh < 255.0f ? (int)fh : 255;
                     while (ql > 0 && decode_q((float)ql, sc, lo) > cl) ql--;
                     while (ql < 255 && decode_q((float)(ql + 1), sc, lo) <= cl) ql++;
                     while (qh < 255 && decode_q((float)qh, sc, lo) < ch) qh++;
