@@ -205,8 +205,8 @@ constexpr uint32_t kStayEighths = 4, kStayAll = 0;
 // SIMDs' issue ports full, so what counts is instructions per visit and lanes per instruction, not
 // fetch latency (eight waves per SIMD cover it).  1080p x 32 frame, closest hits: 26 lanes of 64 active
 // per VALU instruction and 14.0 ms a pass while a wave stayed in its node loop until every lane held a
-// leaf; 38 lanes, a third fewer instructions and 10.1 ms now (the L1 tags are then 62% busy).
-// 2,000,003 closest hits 465 -> 264 us, 300,007 bounded any-hit rays 81 -> 57 us.
+// leaf; 38 lanes, a third fewer instructions and 10.1 ms leaving it early (the L1 tags are then 62% busy).
+// 2,000,003 closest hits 449 -> 271 us, 300,007 bounded any-hit rays 83 -> 61 us.
 //
 // The stack holds the S most recent entries in LDS (slot s at col[s * BLOCK], lanes on distinct
 // banks) and the rest in `spill`; its bottom entry is kSent, so a pop needs no empty check.
